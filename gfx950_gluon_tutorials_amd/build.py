@@ -24,13 +24,13 @@ LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
 # The same kernels with per-workgroup phase stamps (-DG9_TIMING), for
 # profiling.py; never loaded by the wrappers unless G9_LIBRARY points at it.
 LIB_TIMING_PATH = os.path.join(PKG_DIR, "libg9gemm_timing.so")
-SOURCES = ["g9_capi.hip", "g9_fmha.hip"]  # GEMM + MoE + C ABI; flash-attention forward
+SOURCES = ["g9_capi.hip", "g9_tile.hip", "g9_fmha.hip"]  # GEMM + MoE + C ABI; small tiles; flash-attention forward
 # Per-source flags.  g9_fmha.hip: without NaN-preserving semantics for fmax
 # the row-max reduction is one v_max3 per two scores instead of also
 # canonicalizing every MFMA result first (NaN inputs still give NaN rows:
 # their exponentials are NaN).
 SOURCE_FLAGS = {"g9_fmha.hip": ["-fno-honor-nans"]}
-HEADERS = ["g9_common.hpp", "g9_gemm.hpp"]
+HEADERS = ["g9_common.hpp", "g9_gemm.hpp", "g9_tile.hpp", "g9_tile_pick.hpp"]
 
 # -packed-fp32-ops: keep the compiler from forming v_pk_*_f32, whose results
 # have been unreliable on the target machines.

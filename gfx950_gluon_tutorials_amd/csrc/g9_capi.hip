@@ -8,6 +8,7 @@
 
 #include "../../include/gfx950_gemm.h"
 #include "g9_gemm.hpp"
+#include "g9_tile_pick.hpp"
 
 using namespace g9;
 
@@ -219,6 +220,16 @@ int cu_count() {
   return n;
 }
 
+// Row of kTileCost for an operand type, and bytes per operand value.
+int tile_family(int dtype) { return dtype == G9_F16 || dtype == G9_BF16 ? 0 : dtype == G9_BF8 ? 1 : 2; }
+double value_bytes(int dtype) { return tile_family(dtype) == 0 ? 2.0 : dtype == G9_BF8 ? 1.0 : 0.53125; }
+
+// Operand types and wave counts whose 256x256 kernel uses the 16x16 MFMAs of
+// the small tiles, so that both give the same bits.
+bool has_small_tiles(int dtype, int waves) {
+  return waves == 4 || dtype == G9_F16 || dtype == G9_BF16 || dtype == G9_BF8;
+}
+
 bool aligned(const void* p, size_t a) { return ((uintptr_t)p % a) == 0; }
 
 // Workspace layout (both schedules): the header, then a flag region as large
@@ -238,6 +249,16 @@ size_t units_bytes(long long units) {
 size_t splitk_bytes(long long partials) { return units_bytes(2 * partials); }
 size_t streamk_bytes(long long tiles) { return units_bytes(2 * tiles); }
 size_t streamk_half_bytes(long long tiles) { return units_bytes(tiles); }
+
+// Predicted time (us) of split-K with S segments per 256x256 tile: the
+// segment kernel (5 us of launches, a tile's fixed cost, its stages 60% slower
+// than on the half-empty grids the fit is from) and 0.045 us per
+// 256 KiB partial of the reduction.  FP16 512 x 4096 x 8192 (S = 8) measured
+// 37.8 + 11.5 us; 128x64 tiles, whose time this is compared with, 38.1 us.
+double splitk_time(int family, int ns, long long tiles, int S) {
+  const TileCost& c = kTileCost[family][kNumTiles];
+  return 5.0 + c.fixed + 1.6 * c.stage * ((ns + S - 1) / S) + 0.045 * (double)(tiles * S);
+}
 
 // A resolved launch: the kernel (and split-K's reduction), the grid and the
 // parameter block, i.e. everything an entry point works out before it
@@ -278,16 +299,41 @@ int make_plan(int dtype, int out, int schedule, int waves, GemmParams& p, void* 
   p.group_m = kGroupM;
   const long long tiles = (long long)p.tiles_m * p.tiles_n;
   int grid;
+  // Data-parallel launches: the tile with the smallest predicted time.
+  auto data_parallel = [&](int shape) {
+    TileLaunch t;
+    if (shape < kNumTiles && tile_kernel(dtype, shape, t)) {
+      const long long tm = (p.M + t.tm - 1) / t.tm, tn = (p.N + t.tn - 1) / t.tn;
+      if (tm * tn <= INT32_MAX) {
+        p.tiles_m = (int)tm;
+        p.tiles_n = (int)tn;
+        p.out = out == G9_BF16 ? OUT_BF16 : OUT_F16;
+        pl.fn = reinterpret_cast<const void*>(t.fn);
+        pl.block = t.threads;
+        return (int)(tm * tn);
+      }
+    }
+    pl.fn = reinterpret_cast<const void*>(find_kernel(dtype, out, G9_SCHED_DP, waves)->fn);
+    return (int)tiles;
+  };
+  const double bytes = ((double)p.M + p.N) * p.K * value_bytes(dtype) + 2.0 * p.M * p.N;
+  pl.fn = reinterpret_cast<const void*>(k->fn);
   if (schedule == G9_SCHED_SPLITK) {
     const int cus = cu_count();
     if (cus <= 0) return G9_ERR_HIP;
     const int S = g9_splitk_factor(tiles, p.ns, cus);
+    double dp_time = 0;
+    const int shape = has_small_tiles(dtype, waves)
+                          ? pick_tile(tile_family(dtype), p.M, p.N, p.ns, bytes, cus, &dp_time)
+                          : kNumTiles;
     if (S <= 1) {
       // The grid fills the chip (or K is one stage): run the data-parallel kernel.
-      k = find_kernel(dtype, out, G9_SCHED_DP, waves);
-      grid = (int)tiles;
+      grid = data_parallel(shape);
+    } else if (!ws || ws_bytes < splitk_bytes(tiles * S) || !aligned(ws, 256)) {
+      return G9_ERR_WORKSPACE;
+    } else if (shape < kNumTiles && dp_time < splitk_time(tile_family(dtype), p.ns, tiles, S)) {
+      grid = data_parallel(shape);
     } else {
-      if (!ws || ws_bytes < splitk_bytes(tiles * S) || !aligned(ws, 256)) return G9_ERR_WORKSPACE;
       const size_t base = splitk_base(ws_bytes);
       if (base + (size_t)(tiles * S) * kWsTileBytes > ws_bytes) return G9_ERR_WORKSPACE;
       p.ws = reinterpret_cast<float*>(static_cast<char*>(ws) + base);
@@ -298,7 +344,13 @@ int make_plan(int dtype, int out, int schedule, int waves, GemmParams& p, void* 
       pl.red_grid = (int)((threads + 255) / 256);
     }
   } else if (schedule == G9_SCHED_DP) {
-    grid = (int)tiles;
+    int shape = kNumTiles;
+    if (has_small_tiles(dtype, waves)) {
+      const int cus = cu_count();
+      if (cus <= 0) return G9_ERR_HIP;
+      shape = pick_tile(tile_family(dtype), p.M, p.N, p.ns, bytes, cus);
+    }
+    grid = data_parallel(shape);
   } else {
     // The partials go behind the whole flag region g9_workspace_init clears
     // for this workspace size (as split-K's do), so a launch with fewer tiles
@@ -322,7 +374,6 @@ int make_plan(int dtype, int out, int schedule, int waves, GemmParams& p, void* 
   // Last, after every argument check, so bad arguments are reported
   // without touching the HIP runtime.
   if (hipGetDevice(&pl.device) != hipSuccess) return G9_ERR_HIP;
-  pl.fn = reinterpret_cast<const void*>(k->fn);
   pl.grid = grid;
   pl.p = p;
   pl.magic = kPlanMagic;

@@ -150,6 +150,7 @@ struct GemmParams {
                               // the operand resources start that much earlier, stage 0's DMAs zero it
   int tiles_m, tiles_n;
   int num_xcds, group_m;
+  int out;                    // small-tile kernels: output type (OUT_F16, OUT_BF16)
   // stream-K
   float* ws;                  // fp32 partial tiles (256 KiB per tile)
   u32* flags;                 // one flag per tile: (epoch << 16) | stages done
