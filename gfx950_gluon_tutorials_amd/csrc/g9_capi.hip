@@ -302,7 +302,7 @@ int make_plan(int dtype, int out, int schedule, int waves, GemmParams& p, void* 
   // Data-parallel launches: the tile with the smallest predicted time.
   auto data_parallel = [&](int shape) {
     TileLaunch t;
-    if (shape < kNumTiles && tile_kernel(dtype, shape, t)) {
+    if (shape < kNumTiles && tile_kernel(dtype, false, shape, t)) {
       const long long tm = (p.M + t.tm - 1) / t.tm, tn = (p.N + t.tn - 1) / t.tn;
       if (tm * tn <= INT32_MAX) {
         p.tiles_m = (int)tm;
@@ -409,16 +409,28 @@ int launch_moe(int dtype, int out, GemmParams& p, int64_t E, void* stream) {
   const KernelEntry* k = find_moe_kernel(dtype, out);
   if (!k) return G9_ERR_DTYPE;
   if (p.M == 0) return G9_OK;  // no tokens: nothing to write
-  // Upper bound of the experts' m-tiles: sum ceil(M_e / 256) <= ceil(T / 256) + E.
-  const long long tiles_m = (p.M + kTile - 1) / kTile + E;
-  p.tiles_n = (p.N + kTile - 1) / kTile;
+  const int cus = cu_count();
+  if (cus <= 0) return G9_ERR_HIP;
+  TileLaunch t{k->fn, kTile, kTile, 256};
+  int shape = pick_moe_tile(tile_family(dtype), p.M, E, p.N, p.ns, p.K * value_bytes(dtype), cus);
+  if (shape < kNumTiles) {
+    const TileLaunch big = t;
+    tile_kernel(dtype, true, shape, t);
+    if (((p.M + (E < p.M ? E : p.M) * (t.tm - 1)) / t.tm) * ((p.N + t.tn - 1) / t.tn) > INT32_MAX) t = big;
+  }
+  // Upper bound of the experts' m-tiles: sum ceil(M_e / tm) over at most
+  // min(E, T) experts that have rows.
+  const long long rows_e = E < p.M ? E : p.M;
+  const long long tiles_m = ((long long)p.M + rows_e * (t.tm - 1)) / t.tm;
+  p.tiles_n = (p.N + t.tn - 1) / t.tn;
   if (tiles_m * p.tiles_n > INT32_MAX) return G9_ERR_SHAPE;
   p.tiles_m = (int)tiles_m;
   p.num_xcds = kNumXcds;
   p.group_m = kGroupM;
   p.moe_experts = (int)E;
+  p.out = out == G9_BF16 ? OUT_BF16 : OUT_F16;
   void* args[] = {&p};
-  return hipLaunchKernel(reinterpret_cast<const void*>(k->fn), dim3((unsigned)(tiles_m * p.tiles_n)), dim3(256),
+  return hipLaunchKernel(reinterpret_cast<const void*>(t.fn), dim3((unsigned)(tiles_m * p.tiles_n)), dim3(t.threads),
                          args, 0, reinterpret_cast<hipStream_t>(stream)) == hipSuccess
              ? G9_OK
              : G9_ERR_HIP;

@@ -10,8 +10,9 @@ struct TileLaunch {
   TileKernelFn fn;
   int tm, tn, threads;
 };
-// Small-tile kernel `shape` (an index of kTileShapes) of operand type `dtype`.
-bool tile_kernel(int dtype, int shape, TileLaunch& out);
+// Small-tile kernel `shape` (an index of kTileShapes) of operand type `dtype`,
+// dense or grouped.
+bool tile_kernel(int dtype, bool moe, int shape, TileLaunch& out);
 
 // The small tiles, and last the 256x256 kernels' tile.
 constexpr int kNumTiles = 8;
@@ -62,6 +63,26 @@ inline int pick_tile(int family, long long M, long long N, int ns, double bytes,
     }
   }
   if (time) *time = best_t;
+  return best;
+}
+
+// The same for a grouped GEMM of T rows over E experts.  The rows per expert
+// are on the device: an expert is taken to have the average of the experts
+// that can have rows, and half an m-tile more than its rows fill.
+inline int pick_moe_tile(int family, long long T, long long E, long long N, int ns, double row_bytes, int cus) {
+  const double experts = (double)(E < T ? E : T), rows = T / experts;
+  const double bytes = (T + experts * N) * row_bytes + 2.0 * T * N;
+  int best = kNumTiles;
+  double best_t = 0;
+  for (int i = kNumTiles; i >= 0; --i) {
+    const double per = rows / kTileShapes[i][0] + 0.5;
+    const double tiles = experts * (per < 1 ? 1 : per) * (double)((N + kTileShapes[i][1] - 1) / kTileShapes[i][1]);
+    const double t = tile_time(family, i, tiles, ns, bytes, cus) * (i == kNumTiles ? 0.93 : 1.0);
+    if (i == kNumTiles || t < best_t) {
+      best = i;
+      best_t = t;
+    }
+  }
   return best;
 }
 
