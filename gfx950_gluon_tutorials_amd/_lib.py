@@ -81,6 +81,8 @@ SIGNATURES = {
     "g9_workspace_watch": (_int, [_vp, _sz, _vp, _vp]),
     "g9_set_streamk_spin_limit": (ctypes.c_uint32, [ctypes.c_uint32]),
     "g9_transpose_u8": (_int, [_vp, _i64, _i64, _i64, _vp, _i64, _vp]),
+    "g9_quantize_mxfp4": (_int, [_vp, _int, _int, _i64, _vp, _vp, _vp]),
+    "g9_quantize_e5m2": (_int, [_vp, _int, _int, _i64, _vp, _vp, _vp, _vp]),
     "g9_noalloc_error": (_int, [_vp, ctypes.POINTER(_int)]),
     "g9_plan_a16w16": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                               _int, _int, _int, _vp, _sz]),

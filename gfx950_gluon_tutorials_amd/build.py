@@ -24,7 +24,8 @@ LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
 # The same kernels with per-workgroup phase stamps (-DG9_TIMING), for
 # profiling.py; never loaded by the wrappers unless G9_LIBRARY points at it.
 LIB_TIMING_PATH = os.path.join(PKG_DIR, "libg9gemm_timing.so")
-SOURCES = ["g9_capi.hip", "g9_tile.hip", "g9_fmha.hip"]  # GEMM + MoE + C ABI; small tiles; flash-attention forward
+# GEMM + MoE + C ABI; small tiles; operand quantizers; flash-attention forward
+SOURCES = ["g9_capi.hip", "g9_tile.hip", "g9_quant.hip", "g9_fmha.hip"]
 # Per-source flags.  g9_fmha.hip: without NaN-preserving semantics for fmax
 # the row-max reduction is one v_max3 per two scores instead of also
 # canonicalizing every MFMA result first (NaN inputs still give NaN rows:

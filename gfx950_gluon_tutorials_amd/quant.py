@@ -23,6 +23,8 @@ from __future__ import annotations
 
 import torch
 
+from . import _lib
+
 E5M2_MAX = 57344.0
 SCALE_GROUP = 32
 
@@ -30,8 +32,42 @@ SCALE_GROUP = 32
 _E2M1_MIDS = (0.25, 0.75, 1.25, 1.75, 2.5, 3.5, 5.0)
 
 
+_IN = {torch.float16: (16, 0), torch.bfloat16: (16, 1), torch.float32: (32, 0)}
+_SCRATCH_WORDS = 1024
+
+
+def _on_gpu(x: torch.Tensor) -> bool:
+    """Whether x goes to the library's kernels: a plain GPU tensor with values
+    and nothing that follows the torch operations below (a gradient, a
+    forward-mode tangent, vmap, tracing, a dispatch mode)."""
+    return (x.is_cuda and x.numel() > 0 and type(x) in (torch.Tensor, torch.nn.Parameter)
+            and not (x.requires_grad and torch.is_grad_enabled()) and torch.autograd.forward_ad._current_level < 0
+            and not torch._C._functorch.is_functorch_wrapped_tensor(x) and torch._C._len_torch_dispatch_stack() == 0
+            and not torch.compiler.is_compiling() and torch._C._get_tracing_state() is None)
+
+
+def _kernel_input(x: torch.Tensor) -> torch.Tensor:
+    """x's values contiguous, 16-byte aligned and of a type the kernels read."""
+    x = x.detach()
+    if x.dtype not in _IN:
+        x = x.float()
+    x = x.contiguous()
+    return x if x.data_ptr() % 16 == 0 else x.clone()
+
+
 def quantize_e5m2(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """Returns (codes as torch.float8_e5m2, fp32 scale tensor of shape (1,))."""
+    if _on_gpu(x):
+        src = _kernel_input(x)
+        codes = torch.empty(x.shape, dtype=torch.float8_e5m2, device=x.device)
+        scale = torch.empty(1, dtype=torch.float32, device=x.device)
+        scratch = torch.empty(_SCRATCH_WORDS, dtype=torch.int32, device=x.device)
+        with torch.cuda.device(x.device):
+            rc = _lib.load().g9_quantize_e5m2(src.data_ptr(), *_IN[src.dtype], src.numel(), codes.data_ptr(),
+                                              scale.data_ptr(), scratch.data_ptr(),
+                                              torch.cuda.current_stream(x.device).cuda_stream)
+        _lib.check(rc, "g9_quantize_e5m2")
+        return codes, scale
     x = x.float()
     amax = x.abs().amax()
     scale = torch.where(amax > 0, amax / E5M2_MAX, torch.ones_like(amax))
@@ -55,6 +91,15 @@ def quantize_mxfp4(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     if x.dim() != 2 or x.shape[1] % SCALE_GROUP:
         raise ValueError(f"quantize_mxfp4 needs (R, K) with K % 32 == 0, got {tuple(x.shape)}")
     R, K = x.shape
+    if _on_gpu(x):
+        src = _kernel_input(x)
+        packed = torch.empty((R, K // 2), dtype=torch.uint8, device=x.device)
+        scales = torch.empty((R, K // SCALE_GROUP), dtype=torch.uint8, device=x.device)
+        with torch.cuda.device(x.device):
+            rc = _lib.load().g9_quantize_mxfp4(src.data_ptr(), *_IN[src.dtype], R * K // SCALE_GROUP, packed.data_ptr(),
+                                               scales.data_ptr(), torch.cuda.current_stream(x.device).cuda_stream)
+        _lib.check(rc, "g9_quantize_mxfp4")
+        return packed, scales
     g = x.float().reshape(R, K // SCALE_GROUP, SCALE_GROUP)
     amax = g.abs().amax(dim=-1)
     _, ex = torch.frexp(amax)  # amax = m * 2^ex, m in [0.5, 1)

@@ -305,6 +305,20 @@ int g9_transpose_u8(const void* src, int64_t rows, int64_t cols, int64_t src_ld,
                     void* stream);
 
 /*
+ * Operand quantizers: contiguous, 16-byte aligned fp32 (`in_bits` 32), BF16
+ * (16, `bf16` nonzero) or FP16 values.  MXFP4: `groups` groups of 32 values
+ * to 16 bytes each of e2m1 codes (even value in the low nibble) and one E8M0
+ * byte: E = floor(log2(largest magnitude)) - 2, codes rounded to nearest even
+ * and saturated.  BF8: n values to e5m2 codes of x / scale with *scale =
+ * largest magnitude / 57344 (1 for an all-zero tensor); `scratch` holds
+ * G9_QUANT_SCRATCH_WORDS 4-byte words, written and read by the call.
+ */
+#define G9_QUANT_SCRATCH_WORDS 1024
+int g9_quantize_mxfp4(const void* x, int in_bits, int bf16, int64_t groups, void* packed, void* scales, void* stream);
+int g9_quantize_e5m2(const void* x, int in_bits, int bf16, int64_t n, void* codes, void* scale, void* scratch,
+                     void* stream);
+
+/*
  * Name of the kernel a call with this (dtype, out_dtype, schedule, waves)
  * launches (for G9_SCHED_SPLITK: its segment kernel, followed by
  * g9_splitk_reduce_f16 or g9_splitk_reduce_bf16 by output type),
