@@ -53,10 +53,12 @@ def fmha_forward(q, k, v, o, metadata, scale_on_q: bool, variant: int, lse=None)
     strides = get_strides_from_layout(q, k, v, o, metadata)
     arr = [(_lib.ctypes.c_int64 * 4)(*st) for st in strides]
     lib = _lib.load()
-    with torch.cuda.device(dev):
-        stream = torch.cuda.current_stream(dev).cuda_stream
-        rc = lib.g9_fmha_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
-                             lse.data_ptr() if lse is not None else None, batch, nheads_q, nheads_k, S, head_size,
-                             arr[0], arr[1], arr[2], arr[3], float(metadata.sm_scale), _DTYPES[q.dtype],
-                             1 if scale_on_q else 0, variant, stream)
+    args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr() if lse is not None else None, batch,
+            nheads_q, nheads_k, S, head_size, arr[0], arr[1], arr[2], arr[3], float(metadata.sm_scale),
+            _DTYPES[q.dtype], 1 if scale_on_q else 0, variant, torch._C._cuda_getCurrentRawStream(dev.index))
+    if torch._C._cuda_getDevice() == dev.index:
+        rc = lib.g9_fmha_fwd(*args)
+    else:
+        with torch.cuda.device(dev):
+            rc = lib.g9_fmha_fwd(*args)
     _lib.check(rc, "g9_fmha_fwd")

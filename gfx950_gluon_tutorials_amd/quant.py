@@ -55,6 +55,19 @@ def _kernel_input(x: torch.Tensor) -> torch.Tensor:
     return x if x.data_ptr() % 16 == 0 else x.clone()
 
 
+def _call(entry: str, dev: torch.device, *args) -> None:
+    """One launch on the current stream of `dev`."""
+    fn = getattr(_lib.load(), entry)
+    stream = torch._C._cuda_getCurrentRawStream(dev.index)
+    if torch._C._cuda_getDevice() == dev.index:
+        rc = fn(*args, stream)
+    else:
+        with torch.cuda.device(dev):
+            rc = fn(*args, stream)
+    if rc:
+        _lib.check(rc, entry)
+
+
 def quantize_e5m2(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """Returns (codes as torch.float8_e5m2, fp32 scale tensor of shape (1,))."""
     if _on_gpu(x):
@@ -62,11 +75,8 @@ def quantize_e5m2(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         codes = torch.empty(x.shape, dtype=torch.float8_e5m2, device=x.device)
         scale = torch.empty(1, dtype=torch.float32, device=x.device)
         scratch = torch.empty(_SCRATCH_WORDS, dtype=torch.int32, device=x.device)
-        with torch.cuda.device(x.device):
-            rc = _lib.load().g9_quantize_e5m2(src.data_ptr(), *_IN[src.dtype], src.numel(), codes.data_ptr(),
-                                              scale.data_ptr(), scratch.data_ptr(),
-                                              torch.cuda.current_stream(x.device).cuda_stream)
-        _lib.check(rc, "g9_quantize_e5m2")
+        _call("g9_quantize_e5m2", x.device, src.data_ptr(), *_IN[src.dtype], src.numel(), codes.data_ptr(),
+              scale.data_ptr(), scratch.data_ptr())
         return codes, scale
     x = x.float()
     amax = x.abs().amax()
@@ -95,10 +105,8 @@ def quantize_mxfp4(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         src = _kernel_input(x)
         packed = torch.empty((R, K // 2), dtype=torch.uint8, device=x.device)
         scales = torch.empty((R, K // SCALE_GROUP), dtype=torch.uint8, device=x.device)
-        with torch.cuda.device(x.device):
-            rc = _lib.load().g9_quantize_mxfp4(src.data_ptr(), *_IN[src.dtype], R * K // SCALE_GROUP, packed.data_ptr(),
-                                               scales.data_ptr(), torch.cuda.current_stream(x.device).cuda_stream)
-        _lib.check(rc, "g9_quantize_mxfp4")
+        _call("g9_quantize_mxfp4", x.device, src.data_ptr(), *_IN[src.dtype], R * K // SCALE_GROUP, packed.data_ptr(),
+              scales.data_ptr())
         return packed, scales
     g = x.float().reshape(R, K // SCALE_GROUP, SCALE_GROUP)
     amax = g.abs().amax(dim=-1)
