@@ -47,8 +47,9 @@ def _on_gpu(x: torch.Tensor) -> bool:
 
 
 def _kernel_input(x: torch.Tensor) -> torch.Tensor:
-    """x's values contiguous, 16-byte aligned and of a type the kernels read."""
-    x = x.detach()
+    """x's values in memory as they are (no pending negation), contiguous,
+    16-byte aligned and of a type the kernels read."""
+    x = x.detach().resolve_neg()
     if x.dtype not in _IN:
         x = x.float()
     x = x.contiguous()

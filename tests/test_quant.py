@@ -36,3 +36,10 @@ def test_e5m2_matches_oracle(seed, scale):
 def test_mxfp4_rejects_ragged_k():
     with pytest.raises(ValueError):
         Q.quantize_mxfp4(torch.zeros(4, 40))
+
+
+def test_kernel_input_resolves_negation():
+    """The GPU kernels read memory, where a lazily negated view holds the opposite values."""
+    x = torch.randn(2, 32, generator=torch.Generator().manual_seed(0))
+    y = Q._kernel_input(torch._neg_view(x))
+    assert not y.is_neg() and torch.equal(y, -x)
