@@ -302,7 +302,7 @@ int make_plan(int dtype, int out, int schedule, int waves, GemmParams& p, void* 
   // Data-parallel launches: the tile with the smallest predicted time.
   auto data_parallel = [&](int shape) {
     TileLaunch t;
-    if (shape < kNumTiles && tile_kernel(dtype, false, shape, t)) {
+    if (shape < kNumTiles && tile_kernel(dtype, false, shape, t) && tile_addresses(t.tm, p.lda, p.ldsa)) {
       const long long tm = (p.M + t.tm - 1) / t.tm, tn = (p.N + t.tn - 1) / t.tn;
       if (tm * tn <= INT32_MAX) {
         p.tiles_m = (int)tm;
@@ -416,7 +416,9 @@ int launch_moe(int dtype, int out, GemmParams& p, int64_t E, void* stream) {
   if (shape < kNumTiles) {
     const TileLaunch big = t;
     tile_kernel(dtype, true, shape, t);
-    if (((p.M + (E < p.M ? E : p.M) * (t.tm - 1)) / t.tm) * ((p.N + t.tn - 1) / t.tn) > INT32_MAX) t = big;
+    if (!tile_addresses(t.tm, p.lda, p.ldsa) ||
+        ((p.M + (E < p.M ? E : p.M) * (t.tm - 1)) / t.tm) * ((p.N + t.tn - 1) / t.tn) > INT32_MAX)
+      t = big;
   }
   // Upper bound of the experts' m-tiles: sum ceil(M_e / tm) over at most
   // min(E, T) experts that have rows.

@@ -19,6 +19,14 @@ constexpr int kNumTiles = 8;
 constexpr int kTileShapes[kNumTiles + 1][2] = {{16, 16},  {16, 32},   {32, 32},   {64, 32},  {64, 64},
                                                {128, 64}, {128, 128}, {256, 128}, {256, 256}};
 
+// Whether a small tile can address its A rows (lda bytes apart) and row-major
+// A scales (ldsa): its buffer ranges stay below 2^31 bytes, so that dead
+// offsets are out of range.  Row strides go up to 2^24 bytes, which 128 rows
+// allow; the 256-row tile takes them below 2^23.
+inline bool tile_addresses(int tm, long long lda, long long ldsa) {
+  return tm <= 128 || (lda < (1 << 23) && ldsa < (1 << 23));
+}
+
 // Cost of one tile in microseconds, fixed + per K stage (128 bytes of a row),
 // by operand size (16-bit, BF8, MXFP4): the least-squares fit (in the
 // logarithm) of predict() to the kernels' times on 43 shapes from 1 x 1024 to

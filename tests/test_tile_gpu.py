@@ -93,3 +93,44 @@ def test_a4w4_tile_bits(gpu, tile, layout):
     buf, c = _out(gpu, M, N, torch.bfloat16)
     _launch.gemm_a4w4(a, b, sa, sb, c)
     _same(buf, c, want)
+
+
+def _spread(x, stride):
+    """x's rows `stride` bytes apart."""
+    es = x.element_size()
+    buf = torch.empty(x.shape[0] * stride // es, dtype=x.dtype, device=x.device)
+    wide = buf.as_strided(x.shape, (stride // es, 1))
+    wide.copy_(x)
+    return wide
+
+
+# Row strides from where 256 rows stop fitting a 2^31-byte buffer range (the
+# 256x128 tile, which these shapes take with packed rows) to the largest the
+# library takes; K tails need a stride below that.
+@pytest.mark.parametrize("stride", [2**23 - 16, 2**23, 2**24 - 16, 2**24])
+@pytest.mark.parametrize("op", ["f16", "bf8", "mxfp4", "mxfp4_scales"])
+def test_wide_rows(gpu, op, stride):
+    M, N = 1537, 4096
+    K = {"f16": 1024 - 8, "bf8": 1024 - 16}.get(op, 1024)
+    if stride == 2**24 and not op.startswith("mxfp4"):
+        K = 1024
+    print(f"\n[case] wide rows {op} {M}x{N}x{K} stride {stride}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(K)
+    a = torch.randn(M, K, generator=g, device=gpu)
+    b = torch.randn(N, K, generator=g, device=gpu)
+    out = [torch.empty(M, N, dtype=torch.float16, device=gpu) for _ in range(2)]
+    if op == "f16":
+        a, b = a.half(), b.half()
+        for c, x in zip(out, (a, _spread(a, stride))):
+            _launch.gemm_a16w16(x, b.T, c)
+    elif op == "bf8":
+        a, b = a.to(torch.float8_e5m2), b.to(torch.float8_e5m2)
+        for c, x in zip(out, (a, _spread(a, stride))):
+            _launch.gemm_a8w8(x, b.T, c)
+    else:
+        (a, sa), (b, sb) = quant.quantize_mxfp4(a), quant.quantize_mxfp4(b)
+        wide = (a, _spread(sa, stride)) if op == "mxfp4_scales" else (_spread(a, stride), sa)
+        for c, (x, s) in zip(out, ((a, sa), wide)):
+            _launch.gemm_a4w4(x, b, s, sb, c)
+    torch.cuda.synchronize()
+    assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
