@@ -225,8 +225,12 @@ int tile_family(int dtype) { return dtype == G9_F16 || dtype == G9_BF16 ? 0 : dt
 double value_bytes(int dtype) { return tile_family(dtype) == 0 ? 2.0 : dtype == G9_BF8 ? 1.0 : 0.53125; }
 
 // Operand types and wave counts whose 256x256 kernel uses the 16x16 MFMAs of
-// the small tiles, so that both give the same bits.
+// the small tiles, so that both give the same bits.  The timing build keeps to
+// the 256x256 kernels, which carry its phase stamps.
 bool has_small_tiles(int dtype, int waves) {
+#ifdef G9_TIMING
+  return false;
+#endif
   return waves == 4 || dtype == G9_F16 || dtype == G9_BF16 || dtype == G9_BF8;
 }
 
