@@ -1,5 +1,5 @@
 // Small-tile NT GEMM for gfx950: C[M,N] = A[M,K] . B[N,K]^T on output tiles
-// from 16x16 to 128x128, for grids that 256x256 tiles cannot fill the chip
+// from 16x16 to 256x128, for grids that 256x256 tiles cannot fill the chip
 // with (decoding batches, short prompts, experts with few tokens).
 //
 // Every output element is accumulated by the 256x256 kernels' MFMA sequence
