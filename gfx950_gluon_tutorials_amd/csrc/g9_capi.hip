@@ -326,6 +326,13 @@ int make_plan(int dtype, int out, int schedule, int waves, GemmParams& p, void* 
     const int cus = cu_count();
     if (cus <= 0) return G9_ERR_HIP;
     const int S = g9_splitk_factor(tiles, p.ns, cus);
+    // Rows that are no whole number of 128-byte lines apart cost the small
+    // tiles, which read their operands more often, up to twice the predicted
+    // time (BF8 5275 x 512 x 17616: 85.4 us against 57.0 split, at predicted
+    // 0.99 of the split's time; 20 of 33 drawn shapes between 0.7 and 1 lost).
+    // Below 0.65 none of the drawn ones lost.  With whole lines 1 of 12 did
+    // between 0.7 and 1.
+    const bool ragged = p.lda % 128 != 0 || p.ldb % 128 != 0;
     double dp_time = 0;
     const int shape = has_small_tiles(dtype, waves)
                           ? pick_tile(tile_family(dtype), p.M, p.N, p.ns, bytes, cus, &dp_time)
@@ -335,7 +342,7 @@ int make_plan(int dtype, int out, int schedule, int waves, GemmParams& p, void* 
       grid = data_parallel(shape);
     } else if (!ws || ws_bytes < splitk_bytes(tiles * S) || !aligned(ws, 256)) {
       return G9_ERR_WORKSPACE;
-    } else if (shape < kNumTiles && dp_time < splitk_time(tile_family(dtype), p.ns, tiles, S)) {
+    } else if (shape < kNumTiles && dp_time < (ragged ? 0.65 : 1.0) * splitk_time(tile_family(dtype), p.ns, tiles, S)) {
       grid = data_parallel(shape);
     } else {
       const size_t base = splitk_base(ws_bytes);
