@@ -719,10 +719,13 @@ struct Pipe {
         // group row fetch its 128 contiguous bytes and a part reads eight
         // whole 128-byte runs.  Rows past the operand's end read the next
         // group's first rows (scales of A or B rows that read zero, whose
-        // outputs are not stored) or, in the last group, zero.
+        // outputs are not stored) or, in the last group, zero.  The range
+        // ends on a whole dword (lds is one, so it stays inside the group):
+        // the end of a range inside a dword drops that dword, and with it the
+        // scales of the last one to three rows.
         cstride = __builtin_amdgcn_readfirstlane(lds);
         const u32 groups = (u32)p.K / 32;
-        rS = make_rsrc((sa ? p.a_sc : p.b_sc) + hrow, (groups - 1) * lds + (u32)hvalid);
+        rS = make_rsrc((sa ? p.a_sc : p.b_sc) + hrow, (groups - 1) * lds + (((u32)hvalid + 3) & ~3u));
 #pragma unroll
         for (int j = 0; j < SP; ++j) {
           const int grp = 8 * j + (lane >> 3);

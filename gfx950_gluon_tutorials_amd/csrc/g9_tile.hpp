@@ -169,11 +169,12 @@ struct TilePipe {
           cstep[k] = ld;
         } else if constexpr (OpInfo<OP>::kKMajor) {
           // Group G of the chunk: T bytes (one per row) at G * ld; the chunk
-          // lands as 32 group rows of T bytes.
+          // lands as 32 group rows of T bytes.  The range ends on a whole
+          // dword, as in the 256x256 kernels.
           const int per = isa ? T::TM / 16 : T::TN / 16;  // 16-row pieces per group row
           const int piece = 64 * unit + lane;
           const int grp = piece / per, part = piece % per;
-          rs[k] = make_rsrc(base + row0, ((u32)p.K / 32 - 1) * ld + rows);
+          rs[k] = make_rsrc(base + row0, ((u32)p.K / 32 - 1) * ld + ((rows + 3) & ~3u));
           vs[k] = grp < 32 ? (u32)grp * ld + 16u * part : kDeadOff;
           cstep[k] = 32u * ld;
         } else {

@@ -123,6 +123,23 @@ def test_stage_counts_and_ragged_edges(gpu, ns):
     assert R.rel_frobenius(c_km.float().cpu().numpy(), ref) <= 1e-3
 
 
+@pytest.mark.parametrize("schedule", ["dp", "streamk", "splitk"])
+@pytest.mark.parametrize("M,N,K", [(3, 9, 1024), (37, 50, 512), (129, 255, 768), (301, 267, 2304), (517, 1798, 1536),
+                                   (1671, 1165, 1536), (4099, 4093, 768)])
+def test_row_counts_off_dwords(gpu, M, N, K, schedule):
+    """Row counts that are no multiple of 4: the last group's last rows share a
+    dword with padding.  Bit-equal to the row-major scales on small and 256x256
+    tiles, whole and split."""
+    _say(f"a4w4 K-major, rows off dwords {M}x{N}x{K} {schedule}")
+    gen = torch.Generator().manual_seed(M + N)
+    pa, sa = (t.to(gpu) for t in quant.quantize_mxfp4(torch.randn(M, K, generator=gen)))
+    pb, sb = (t.to(gpu) for t in quant.quantize_mxfp4(torch.randn(N, K, generator=gen)))
+    rm = _run(gpu, pa, pb, sa, sb, schedule=schedule)
+    km = _run(gpu, pa, pb, _kmajor(sa, pad_rows=-M % 4), _kmajor(sb, pad_rows=4 + -N % 4), schedule=schedule)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(_bits(km), _bits(rm))
+
+
 @pytest.mark.parametrize("M,N,K", [(3840, 3840, 4096), (1280, 2304, 2560)])
 def test_streamk_and_splitk(gpu, M, N, K):
     _say(f"a4w4 K-major stream-K / split-K {M}x{N}x{K}")
