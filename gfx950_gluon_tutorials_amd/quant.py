@@ -56,6 +56,19 @@ def _kernel_input(x: torch.Tensor) -> torch.Tensor:
     return x if x.data_ptr() % 16 == 0 else x.clone()
 
 
+def _e5m2_buffers(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    """(values, codes) of one shape and one dense layout, so that the kernel
+    can walk both as flat arrays.  The codes have the strides of a torch
+    elementwise result, x's own where x is dense: the codes of w.t() are the
+    K-contiguous (K, N) view that the BF8 GEMM reads in place."""
+    x = x.detach().resolve_neg()
+    codes = torch.empty_like(x, dtype=torch.float8_e5m2)
+    if x.dtype in _IN and x.stride() == codes.stride() and x.data_ptr() % 16 == 0:
+        return x, codes
+    dtype = x.dtype if x.dtype in _IN else torch.float32
+    return torch.empty_strided(x.shape, codes.stride(), dtype=dtype, device=x.device).copy_(x), codes
+
+
 def _call(entry: str, dev: torch.device, *args) -> None:
     """One launch on the current stream of `dev`."""
     fn = getattr(_lib.load(), entry)
@@ -72,8 +85,7 @@ def _call(entry: str, dev: torch.device, *args) -> None:
 def quantize_e5m2(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """Returns (codes as torch.float8_e5m2, fp32 scale tensor of shape (1,))."""
     if _on_gpu(x):
-        src = _kernel_input(x)
-        codes = torch.empty(x.shape, dtype=torch.float8_e5m2, device=x.device)
+        src, codes = _e5m2_buffers(x)
         scale = torch.empty(1, dtype=torch.float32, device=x.device)
         scratch = torch.empty(_SCRATCH_WORDS, dtype=torch.int32, device=x.device)
         _call("g9_quantize_e5m2", x.device, src.data_ptr(), *_IN[src.dtype], src.numel(), codes.data_ptr(),

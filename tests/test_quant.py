@@ -1,6 +1,8 @@
 """The product's torch quantizers agree bit for bit with the oracle's numpy
 restatement (CPU tensors)."""
 
+import itertools
+
 import numpy as np
 import pytest
 import torch
@@ -43,3 +45,32 @@ def test_kernel_input_resolves_negation():
     x = torch.randn(2, 32, generator=torch.Generator().manual_seed(0))
     y = Q._kernel_input(torch._neg_view(x))
     assert not y.is_neg() and torch.equal(y, -x)
+
+
+def _layouts():
+    """3-D and 2-D views: every order of dimensions, dense, sliced, stepped, broadcast, shifted off the 16-byte grid."""
+    g = torch.Generator().manual_seed(1)
+    r = lambda *shape: torch.randn(*shape, generator=g)
+    for p in itertools.permutations(range(3)):
+        yield r(3, 4, 8).permute(p)
+        yield r(3, 1, 8).permute(p)
+        yield r(3, 4, 16)[:, :, :8].permute(p)
+        yield r(3, 4, 16)[:, :, ::2].permute(p)
+        yield r(3, 1, 8).expand(3, 4, 8).permute(p)
+    yield r(6, 8).t()
+    yield r(6, 8)[:, 2:3]
+    yield r(1 + 48)[1:].reshape(6, 8).t()
+    yield r(2, 3, 4, 5).contiguous(memory_format=torch.channels_last)
+    yield torch._neg_view(r(6, 8).t())
+    yield r(1)[0]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16, torch.float64])
+def test_e5m2_buffers_keep_the_layout_of_the_torch_operations(dtype):
+    for x in _layouts():
+        x = torch._neg_view(torch._neg_view(x).to(dtype)) if x.is_neg() else x.to(dtype)
+        src, codes = Q._e5m2_buffers(x)
+        want, _ = Q.quantize_e5m2(x)  # on the CPU: the torch operations
+        assert codes.shape == want.shape and codes.stride() == want.stride(), (x.shape, x.stride())
+        assert src.stride() == codes.stride() and src.dtype in Q._IN and src.data_ptr() % 16 == 0
+        assert not src.is_neg() and torch.equal(src, x.to(src.dtype))

@@ -7,6 +7,8 @@ import pytest
 import torch
 
 from gfx950_gluon_tutorials_amd import quant
+from gfx950_gluon_tutorials_amd.gemm import _launch
+from gfx950_gluon_tutorials_amd.gemm.prepared import PreparedGemm
 
 pytestmark = pytest.mark.gpu
 
@@ -22,6 +24,7 @@ def _check(x):
             continue
         got, want = fn(x), [t.as_subclass(torch.Tensor) for t in fn(y)]
         assert got[0].dtype == want[0].dtype and got[1].shape == want[1].shape
+        assert got[0].stride() == want[0].stride()
         assert torch.equal(got[0].view(torch.uint8), want[0].view(torch.uint8))
         assert torch.equal(got[1].view(bits), want[1].view(bits))
 
@@ -81,3 +84,18 @@ def test_quantizers_leave_followed_tensors_to_torch(gpu):
     with torch.autograd.forward_ad.dual_level():
         d = torch.autograd.forward_ad.make_dual(w[0], torch.ones_like(w[0]))
         assert torch.autograd.forward_ad.unpack_dual(quant.quantize_e5m2(d)[1]).tangent is not None
+
+
+def test_e5m2_of_a_transposed_weight_is_read_in_place(gpu):
+    """The codes of w.t() keep its strides, so they are the (K, N) operand of the
+    BF8 GEMM as they are (a prepared launch refuses one that needs a copy)."""
+    a, sa = quant.quantize_e5m2(torch.randn(48, 256, device=gpu))
+    w = torch.randn(96, 256, device=gpu)
+    b, sb = quant.quantize_e5m2(w.t())
+    nk, sn = quant.quantize_e5m2(w)
+    assert b.stride() == (1, 256) and torch.equal(b.t().view(torch.uint8), nk.view(torch.uint8)) and torch.equal(sb, sn)
+    c, want = (torch.empty(48, 96, dtype=torch.bfloat16, device=gpu) for _ in range(2))
+    PreparedGemm.a8w8([(a, b, c, sa, sb)])()
+    _launch.gemm_a8w8(a, nk.t(), want, a_scale=sa, b_scale=sb)
+    torch.cuda.synchronize()
+    assert torch.equal(c, want)
