@@ -1560,67 +1560,97 @@ G9_DEV void gemm_dp(const GemmParams& p) {
 
 // Grouped ("MoE") GEMM over E experts: expert e multiplies rows
 // [off[e], off[e+1]) of A (tokens sorted by expert) by its own B_e (for BF8
-// with its own fp32 scale b_scale[e]) into the same rows of C.  The grid covers tiles_m x tiles_n tiles with tiles_m an
-// upper bound of the experts' m-tiles (sum of ceil(M_e / 256) <= ceil(M / 256)
-// + E); each workgroup finds the expert of its m-tile and then runs the
-// data-parallel tile unchanged on that expert's rows and weights.  Workgroups
+// with its own fp32 scale b_scale[e]) into the same rows of C.  The grid covers
+// tiles_m x tiles_n tiles with tiles_m an upper bound of the experts' m-tiles
+// (at most min(E, M) of them have rows: sum of ceil(M_e / TILE) <=
+// floor((M + min(E, M) (TILE - 1)) / TILE)); each workgroup finds the expert of
+// its m-tile and then runs the data-parallel tile unchanged on that expert's
+// rows and weights.  Workgroups
 // past the last expert's tiles exit.  Offsets are clamped to [0, M] (and each
 // expert's end to at least its start), so any offset table keeps every access
 // inside A, C and the experts' B.
 
-// The tile of workgroup `bid`: 64 experts per pass, one per lane.  A first
-// pass counts the experts' TILE-row m-tiles, so that the workgroups that have
-// a tile are the first total * tiles_n ones and tile_coords spreads exactly
-// those over the XCDs (with the host's upper bound in its place the unused
-// tiles all fell to the last XCDs: MXFP4, 32 experts, 32768 tokens, 512 -> 494
-// us; BF16, 128 tokens over the same experts, 392 -> 307 us).  The second finds the expert of the m-tile (an inclusive wave
-// prefix sum of the counts, a ballot for the lane whose range holds it).
-// Returns false for workgroups past the last tile.
+// The tile of workgroup `bid`.  Each lane counts the TILE-row m-tiles of its
+// ceil(E / 64) consecutive experts; a wave prefix sum gives their total, so
+// that the workgroups that have a tile are the first total * tiles_n ones and
+// tile_coords spreads exactly those over the XCDs (with the host's upper bound
+// in its place the unused tiles all fell to the last XCDs: MXFP4, 32 experts,
+// 32768 tokens, 512 -> 494 us).  The first lane whose range ends past the
+// m-tile has its expert; with more than 64 experts a second pass, one of that
+// lane's experts per lane, finds which.  A workgroup waits for these loads and
+// sums before its first DMA, so their number counts where tiles are short: one
+// pass over all experts, 64 at a time, and a second up to the expert took MXFP4
+// 512 experts, 8192 tokens, N 1024, K 2048 230 us, two passes 166; with 256
+// experts 90 and 88.  Sums saturate at tiles_m, which bounds those of every
+// valid table, so no table leads past an expert's own tiles.  Returns false for
+// workgroups past the last tile.
 template <int TILE>
 G9_DEV bool moe_find(const GemmParams& p, int bid, int& expert, int& tm, int& tn, int& row0, int& rows) {
   const int lane = threadIdx.x & 63;
-  const int T = p.M, E = p.moe_experts;
-  int lo = 0, hi = 0, n = 0, incl = 0;
-  auto scan = [&](int e) {
-    lo = hi = n = 0;
-    if (e < E) {
-      lo = min(max(p.moe_off[e], 0), T);
-      hi = min(max(p.moe_off[e + 1], lo), T);
-      n = (hi - lo + TILE - 1) / TILE;
-    }
-    incl = n;
+  const int T = p.M, E = p.moe_experts, cap = p.tiles_m;
+  int lo, hi;
+  // m-tiles of the expert between offsets `first` and `last`, and its rows lo .. hi - 1.
+  auto count = [&](int first, int last) {
+    lo = min(max(first, 0), T);
+    hi = min(max(last, lo), T);
+    return (hi - lo + TILE - 1) / TILE;
+  };
+  auto prefix = [&](int n) {
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
-      const int v = __shfl_up(incl, d, 64);
-      if (lane >= d) incl += v;
+      const int v = __shfl_up(n, d, 64);
+      if (lane >= d) n = min(n + v, cap);
     }
+    return n;
   };
-  int total = 0;
-  for (int e0 = 0; e0 < E; e0 += 64) {
-    scan(e0 + lane);
-    // tiles_m bounds the sum of every valid table.
-    total = min(total + __builtin_amdgcn_readfirstlane(__shfl(incl, 63, 64)), p.tiles_m);
+  // Experts past the last one are empty: both their offsets are off[E].
+  auto offset = [&](int e) { return p.moe_off[min(e, E)]; };
+  const int per = (E + 63) / 64;
+  int incl = 0;
+  if (per == 1) {
+    incl = count(offset(lane), offset(lane + 1));
+  } else {
+    // Eight experts at a time, so that their loads are in flight together.
+    constexpr int kBatch = 8;
+    for (int k = 0; k < per; k += kBatch) {
+      int v[kBatch + 1];
+#pragma unroll
+      for (int i = 0; i <= kBatch; ++i) v[i] = offset(lane * per + min(k + i, per));
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) incl = min(incl + (k + i < per ? count(v[i], v[i + 1]) : 0), cap);
+    }
   }
+  incl = prefix(min(incl, cap));
+  const int total = __builtin_amdgcn_readfirstlane(__shfl(incl, 63, 64));
   const int tiles = total * p.tiles_n;
   if (bid >= tiles) return false;
   int mt;
   tile_coords(bid, tiles, total, p.tiles_n, p.num_xcds, p.group_m, mt, tn);
-  int base = 0;
-  for (int e0 = 0; e0 < E; e0 += 64) {
-    if (E > 64) scan(e0 + lane);
-    const int first = base + incl - n;
-    const unsigned long long hit = __ballot(n > 0 && mt >= first && mt < base + incl);
-    if (hit) {
-      const int l = __ffsll((long long)hit) - 1;
-      expert = __builtin_amdgcn_readfirstlane(e0 + l);
-      tm = __builtin_amdgcn_readfirstlane(mt - __shfl(first, l, 64));
-      row0 = __builtin_amdgcn_readfirstlane(__shfl(lo, l, 64));
-      rows = __builtin_amdgcn_readfirstlane(__shfl(hi - lo, l, 64));
-      return true;
+  // The lane whose range holds m-tile mt, which becomes its place in the range.
+  auto owner = [&]() {
+    const int l = __ffsll((long long)__ballot(incl > mt)) - 1;
+    if (l > 0) mt -= __builtin_amdgcn_readfirstlane(__shfl(incl, l - 1, 64));
+    return l;
+  };
+  int l = owner();
+  expert = l * per;
+  if (per > 1) {
+    int k = 0;
+    for (; k < per; k += 64) {
+      const int e = expert + k + lane;
+      incl = prefix(k + lane < per ? min(count(offset(e), offset(e + 1)), cap) : 0);
+      const int sum = __builtin_amdgcn_readfirstlane(__shfl(incl, 63, 64));
+      if (mt < sum) break;
+      mt -= sum;
     }
-    base += __shfl(incl, 63, 64);
+    if (k >= per) return false;  // only if the table changed between the passes
+    l = owner();
+    expert += k + l;
   }
-  return false;
+  tm = mt;
+  row0 = __builtin_amdgcn_readfirstlane(__shfl(lo, l, 64));
+  rows = __builtin_amdgcn_readfirstlane(__shfl(hi - lo, l, 64));
+  return true;
 }
 
 // The parameters of expert `expert`'s own GEMM: rows row0 .. row0 + rows - 1

@@ -1,8 +1,9 @@
 """CPU checks of the grouped (MoE) GEMM: argument validation of the C ABI
 (status codes returned before any launch), kernel names, and a restatement
-of the kernel's expert lookup (g9_gemm.hpp moe_find) showing that any offset
-table keeps every access inside A, C and the experts' B, and that valid tables
-give each expert's rows to exactly one tile."""
+of the kernel's expert lookup (g9_gemm.hpp moe_find, with the grid of
+g9_capi.hip launch_moe) at every tile height, with up to and past one expert
+per lane, showing that any offset table keeps every access inside A, C and the
+experts' B, and that valid tables give each expert's rows to exactly one tile."""
 
 import numpy as np
 import pytest
@@ -71,57 +72,115 @@ def test_moe_kernel_names():
     assert _lib.moe_kernel_name(_lib.G9_F16, _lib.G9_BF16) is None
 
 
-def moe_find(off, E, T, mt):
-    """Restatement of the kernel's lookup: clamp each expert's [lo, hi) into [0, T], count its 256-row
-    tiles, and return (expert, local m-tile, lo, rows) of m-tile mt, or None."""
-    base = 0
-    for e in range(E):
-        lo = min(max(int(off[e]), 0), T)
-        hi = min(max(int(off[e + 1]), lo), T)
-        n = (hi - lo + 255) // 256
-        if n and base <= mt < base + n:
-            return e, mt - base, lo, hi - lo
-        base += n
-    return None
+TILES = [16, 32, 64, 128, 256]
+XCDS, GROUP_M = 8, 4
 
 
-def test_moe_lookup_covers_valid_tables_exactly_once():
-    rng = np.random.default_rng(0)
-    for _ in range(200):
-        E = int(rng.integers(1, 20))
-        counts = rng.integers(0, 700, E)
+def grid_m(T, E, tile):
+    """The launch's m-tiles (g9_capi.hip launch_moe): at most min(E, T) experts have rows."""
+    return (T + min(E, T) * (tile - 1)) // tile
+
+
+def tile_coords(pid, grid, tiles_m, tiles_n):
+    """Restatement of g9_common.hpp tile_coords: contiguous ranges to XCDs, then groups of GROUP_M m-tiles."""
+    per, tall = -(-grid // XCDS), grid % XCDS or XCDS
+    xcd, local = pid % XCDS, pid // XCDS
+    pid = xcd * per + local if xcd < tall else tall * per + (xcd - tall) * (per - 1) + local
+    first = pid // (GROUP_M * tiles_n) * GROUP_M
+    size = min(tiles_m - first, GROUP_M)
+    r = pid % (GROUP_M * tiles_n)
+    return first + r % size, r // size
+
+
+def moe_find(off, E, T, tile, cap, tiles_n, bid, lanes=64):
+    """Restatement of the kernel's lookup with `lanes` lanes: every lane counts its consecutive experts, the first
+    whose saturating prefix sum passes the m-tile owns it, and a second pass finds the expert among its own.
+    Returns (expert, m-tile of the expert, n-tile, first row, rows), or None past the last tile."""
+    def count(e):
+        lo = min(max(int(off[min(e, E)]), 0), T)
+        hi = min(max(int(off[min(e + 1, E)]), lo), T)
+        return lo, hi, -(-(hi - lo) // tile)
+
+    def prefix(ns):
+        out, s = [], 0
+        for n in ns:
+            s = min(s + n, cap)
+            out.append(s)
+        return out
+
+    def owner(incl, mt):
+        lane = next(i for i, s in enumerate(incl) if s > mt)
+        return lane, mt - (incl[lane - 1] if lane else 0)
+
+    per = -(-E // lanes)
+    incl = prefix([min(sum(count(lane * per + k)[2] for k in range(per)), cap) for lane in range(lanes)])
+    total = incl[-1]
+    if bid >= total * tiles_n:
+        return None
+    mt, tn = tile_coords(bid, total * tiles_n, total, tiles_n)
+    lane, mt = owner(incl, mt)
+    e = lane * per
+    for k in range(0, per, lanes) if per > 1 else ():
+        incl = prefix([min(count(e + k + i)[2], cap) if k + i < per else 0 for i in range(lanes)])
+        if mt < incl[-1]:
+            lane, mt = owner(incl, mt)
+            e += k + lane
+            break
+        mt -= incl[-1]
+    else:
+        assert per == 1
+    lo, hi, _ = count(e)
+    return e, mt, tn, lo, hi - lo
+
+
+# (experts, lanes): one expert per lane, several, and more than one pass over a lane's own.
+LOOKUPS = [(1, 64), (20, 64), (64, 64), (65, 64), (70, 64), (300, 64), (30, 4), (90, 4)]
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("E,lanes", LOOKUPS)
+def test_moe_lookup_covers_valid_tables_exactly_once(E, lanes, tile):
+    """Every workgroup of the grid that has a tile has its own, and together they are the experts' rows."""
+    rng = np.random.default_rng(E * tile)
+    for mean, tiles_n in ((3, 2), (tile, 1), (2 * tile, 3)):
+        counts = rng.integers(0, 2 * min(mean, 60_000 // E) + 1, E)
         counts[rng.random(E) < 0.3] = 0
         off = np.concatenate([[0], np.cumsum(counts)])
         T = int(off[-1]) + int(rng.integers(0, 300))
-        bound = -(-T // 256) + E
-        owner = np.full(T, -1)
-        for mt in range(bound):
-            r = moe_find(off, E, T, mt)
+        bound = grid_m(T, E, tile)
+        seen, rows = set(), np.zeros(T, dtype=int)
+        real = int(np.sum(-(-counts // tile)))
+        assert real <= bound
+        bids = range(bound * tiles_n) if real <= 300 else sorted(rng.choice(bound * tiles_n, 300, replace=False))
+        for bid in bids:
+            r = moe_find(off, E, T, tile, bound, tiles_n, int(bid), lanes)
+            assert (r is None) == (bid >= real * tiles_n)
             if r is None:
                 continue
-            e, lt, lo, rows = r
-            assert 0 <= lt < -(-rows // 256)
-            sl = slice(lo + 256 * lt, lo + min(256 * (lt + 1), rows))
-            assert np.all(owner[sl] == -1)  # no row is computed twice
-            owner[sl] = e
-        for e in range(E):
-            assert np.all(owner[off[e]:off[e + 1]] == e)
-        assert np.all(owner[off[-1]:] == -1)
+            e, mt, tn, lo, n = r
+            assert lo == off[e] and n == counts[e] and 0 <= mt < -(-n // tile) and 0 <= tn < tiles_n
+            assert (e, mt, tn) not in seen
+            seen.add((e, mt, tn))
+            rows[lo + tile * mt:lo + min(tile * (mt + 1), n)] += tn == 0
+        if len(bids) == bound * tiles_n:
+            assert len(seen) == real * tiles_n
+            assert np.all(rows[:off[-1]] == 1) and np.all(rows[off[-1]:] == 0)
 
 
-def test_moe_lookup_keeps_garbage_tables_in_bounds():
-    rng = np.random.default_rng(1)
-    for _ in range(300):
-        E = int(rng.integers(1, 70))
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("E,lanes", LOOKUPS)
+def test_moe_lookup_keeps_garbage_tables_in_bounds(E, lanes, tile):
+    rng = np.random.default_rng(E + tile)
+    for _ in range(6):
         T = int(rng.integers(1, 3000))
         off = rng.integers(-5000, 8000, E + 1)
-        bound = -(-T // 256) + E
-        for mt in range(bound):
-            r = moe_find(off, E, T, mt)
+        bound = grid_m(T, E, tile)
+        for bid in rng.integers(0, bound * 2, 60):
+            r = moe_find(off, E, T, tile, bound, 2, int(bid), lanes)
             if r is None:
                 continue
-            e, lt, lo, rows = r
-            assert 0 <= e < E and 0 <= lo and lo + rows <= T
+            e, mt, tn, lo, rows = r
+            assert 0 <= e < E and 0 <= tn < 2 and 0 <= lo and lo + rows <= T
             # rows the tile reads from A and writes to C
-            first, last = lo + 256 * lt, lo + min(256 * (lt + 1), rows)
+            first, last = lo + tile * mt, lo + min(tile * (mt + 1), rows)
             assert 0 <= first < last <= T

@@ -58,3 +58,25 @@ def test_moe_tile_bits(gpu, kind, E, mean, N, K):
             assert torch.equal(c[r].view(torch.int16), want.view(torch.int16)), f"expert {e}"
     torch.cuda.synchronize()
     assert torch.all(c[int(off[-1]):] == 7.0)
+
+
+@pytest.mark.parametrize("E", [64, 65, 512, 577, 4097, 5000])
+def test_many_experts(gpu, E):
+    """One expert per lane of the lookup, several, more than its batch of loads and more than
+    64 (a second pass of more than one chunk), with empty experts: small integers, whose
+    products are exact, against torch in fp32."""
+    T, N, K = 2 * E + 3, 24, 64
+    print(f"\n[case] moe f16 E={E} T={T} N={N} K={K}", flush=True)
+    rng = np.random.default_rng(E)
+    counts = rng.multinomial(2 * E, rng.dirichlet([0.5] * E))
+    owner = torch.from_numpy(np.repeat(np.arange(E), counts)).to(gpu)
+    offs = torch.from_numpy(np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)).to(gpu)
+    g = torch.Generator(device=gpu).manual_seed(E)
+    a = torch.randint(-2, 3, (T, K), generator=g, device=gpu).half()
+    b = torch.randint(-2, 3, (E, N, K), generator=g, device=gpu).half()
+    c = torch.full((T, N), 7.0, dtype=torch.float16, device=gpu)
+    moe_matmul(a, b, offs, c)
+    want = (a[:2 * E, None].float() * b[owner].float()).sum(-1)
+    torch.cuda.synchronize()
+    assert torch.equal(c[:2 * E].float(), want)
+    assert torch.all(c[2 * E:] == 7.0)
