@@ -722,10 +722,12 @@ struct Pipe {
         // outputs are not stored) or, in the last group, zero.  The range
         // ends on a whole dword (lds is one, so it stays inside the group):
         // the end of a range inside a dword drops that dword, and with it the
-        // scales of the last one to three rows.
+        // scales of the last one to three rows.  A half tile with no valid row
+        // has an empty range: its base lies up to 127 bytes past the last row,
+        // so that the last group's bytes would end past the array.
         cstride = __builtin_amdgcn_readfirstlane(lds);
         const u32 groups = (u32)p.K / 32;
-        rS = make_rsrc((sa ? p.a_sc : p.b_sc) + hrow, (groups - 1) * lds + (((u32)hvalid + 3) & ~3u));
+        rS = make_rsrc((sa ? p.a_sc : p.b_sc) + hrow, hvalid ? (groups - 1) * lds + (((u32)hvalid + 3) & ~3u) : 0u);
 #pragma unroll
         for (int j = 0; j < SP; ++j) {
           const int grp = 8 * j + (lane >> 3);

@@ -269,3 +269,21 @@ def test_transpose_writes_are_bank_conflict_free_per_8_lanes():
         g, a2, b = lane >> 4, (lane >> 3) & 1, lane & 7
         old.append(32 * (2 * (g ^ (2 * a2)) + (b >> 2) + 8 * (b & 3)) + 16 * (a2 ^ (b & 1)))
     assert any(len(set(_banks(old[p0:p0 + 8], width=16))) < 32 for p0 in range(0, 64, 8))
+
+
+@pytest.mark.parametrize("half", [128, 16, 32, 64, 256])
+def test_k_major_ranges_hold_every_valid_row_and_stay_inside_the_array(half):
+    """The buffer range of a K-major scale array, restated: from the first row of a tile (of a half tile of 128 rows in
+    the 256x256 kernels, where it may lie past the last row), (groups - 1) strides and the valid rows rounded up to
+    whole dwords, nothing where no row is valid.  Every dword that holds a valid scale is inside it, and it ends
+    inside the array, whose groups are a multiple of 4 bytes apart."""
+    groups = 8
+    for rows in list(range(1, 70)) + [127, 128, 129, 255, 256, 257, 300, 511, 515]:
+        for ld in {-(-rows // 4) * 4, -(-rows // 4) * 4 + 4, rows // 256 * 256 + 256}:
+            tile = 256 if half == 128 else half
+            for base in range(0, -(-rows // tile) * tile, half):
+                valid = min(max(rows - base, 0), half)
+                end = (groups - 1) * ld + (valid + 3) // 4 * 4 if valid else 0
+                assert end == 0 or base + end <= groups * ld
+                last = (groups - 1) * ld + valid - 1
+                assert valid == 0 or last // 4 * 4 + 4 <= end
