@@ -254,16 +254,6 @@ size_t splitk_bytes(long long partials) { return units_bytes(2 * partials); }
 size_t streamk_bytes(long long tiles) { return units_bytes(2 * tiles); }
 size_t streamk_half_bytes(long long tiles) { return units_bytes(tiles); }
 
-// Predicted time (us) of split-K with S segments per 256x256 tile: the
-// segment kernel (5 us of launches, a tile's fixed cost, its stages 60% slower
-// than on the half-empty grids the fit is from) and 0.045 us per
-// 256 KiB partial of the reduction.  FP16 512 x 4096 x 8192 (S = 8) measured
-// 37.8 + 11.5 us; 128x64 tiles, whose time this is compared with, 38.1 us.
-double splitk_time(int family, int ns, long long tiles, int S) {
-  const TileCost& c = kTileCost[family][kNumTiles];
-  return 5.0 + c.fixed + 1.6 * c.stage * ((ns + S - 1) / S) + 0.045 * (double)(tiles * S);
-}
-
 // A resolved launch: the kernel (and split-K's reduction), the grid and the
 // parameter block, i.e. everything an entry point works out before it
 // enqueues.  g9_plan_* keep it in the caller's g9_plan; run_plan only
@@ -306,43 +296,36 @@ int make_plan(int dtype, int out, int schedule, int waves, GemmParams& p, void* 
   // Data-parallel launches: the tile with the smallest predicted time.
   auto data_parallel = [&](int shape) {
     TileLaunch t;
-    if (shape < kNumTiles && tile_kernel(dtype, false, shape, t) && tile_addresses(t.tm, p.lda, p.ldsa)) {
-      const long long tm = (p.M + t.tm - 1) / t.tm, tn = (p.N + t.tn - 1) / t.tn;
-      if (tm * tn <= INT32_MAX) {
-        p.tiles_m = (int)tm;
-        p.tiles_n = (int)tn;
-        p.out = out == G9_BF16 ? OUT_BF16 : OUT_F16;
-        pl.fn = reinterpret_cast<const void*>(t.fn);
-        pl.block = t.threads;
-        return (int)(tm * tn);
-      }
+    if (shape < kNumTiles && tile_kernel(dtype, false, shape, t)) {
+      p.tiles_m = (p.M + t.tm - 1) / t.tm;
+      p.tiles_n = (p.N + t.tn - 1) / t.tn;
+      p.out = out == G9_BF16 ? OUT_BF16 : OUT_F16;
+      pl.fn = reinterpret_cast<const void*>(t.fn);
+      pl.block = t.threads;
+      return p.tiles_m * p.tiles_n;
     }
     pl.fn = reinterpret_cast<const void*>(find_kernel(dtype, out, G9_SCHED_DP, waves)->fn);
     return (int)tiles;
   };
-  const double bytes = ((double)p.M + p.N) * p.K * value_bytes(dtype) + 2.0 * p.M * p.N;
+  TileProblem problem{tile_family(dtype), p.M, p.N, p.ns, ((double)p.M + p.N) * p.K * value_bytes(dtype) + 2.0 * p.M * p.N,
+                      p.lda, p.ldsa, 0};
+  auto small_tile = [&](int cus) {
+    problem.cus = cus;
+    return has_small_tiles(dtype, waves) ? pick_tile(problem) : kNumTiles;
+  };
   pl.fn = reinterpret_cast<const void*>(k->fn);
   if (schedule == G9_SCHED_SPLITK) {
     const int cus = cu_count();
     if (cus <= 0) return G9_ERR_HIP;
     const int S = g9_splitk_factor(tiles, p.ns, cus);
-    // Rows that are no whole number of 128-byte lines apart cost the small
-    // tiles, which read their operands more often, up to twice the predicted
-    // time (BF8 5275 x 512 x 17616: 85.4 us against 57.0 split, at predicted
-    // 0.99 of the split's time; 20 of 33 drawn shapes between 0.7 and 1 lost).
-    // Below 0.65 none of the drawn ones lost.  With whole lines 1 of 12 did
-    // between 0.7 and 1.
+    const int shape = small_tile(cus);
     const bool ragged = p.lda % 128 != 0 || p.ldb % 128 != 0;
-    double dp_time = 0;
-    const int shape = has_small_tiles(dtype, waves)
-                          ? pick_tile(tile_family(dtype), p.M, p.N, p.ns, bytes, cus, &dp_time)
-                          : kNumTiles;
     if (S <= 1) {
       // The grid fills the chip (or K is one stage): run the data-parallel kernel.
       grid = data_parallel(shape);
     } else if (!ws || ws_bytes < splitk_bytes(tiles * S) || !aligned(ws, 256)) {
       return G9_ERR_WORKSPACE;
-    } else if (shape < kNumTiles && dp_time < (ragged ? 0.65 : 1.0) * splitk_time(tile_family(dtype), p.ns, tiles, S)) {
+    } else if (tile_beats_split(problem, shape, tiles, S, ragged)) {
       grid = data_parallel(shape);
     } else {
       const size_t base = splitk_base(ws_bytes);
@@ -359,7 +342,7 @@ int make_plan(int dtype, int out, int schedule, int waves, GemmParams& p, void* 
     if (has_small_tiles(dtype, waves)) {
       const int cus = cu_count();
       if (cus <= 0) return G9_ERR_HIP;
-      shape = pick_tile(tile_family(dtype), p.M, p.N, p.ns, bytes, cus);
+      shape = small_tile(cus);
     }
     grid = data_parallel(shape);
   } else {
@@ -423,17 +406,14 @@ int launch_moe(int dtype, int out, GemmParams& p, int64_t E, void* stream) {
   const int cus = cu_count();
   if (cus <= 0) return G9_ERR_HIP;
   TileLaunch t{k->fn, kTile, kTile, 256};
-  int shape = pick_moe_tile(tile_family(dtype), p.M, E, p.N, p.ns, p.K * value_bytes(dtype), cus);
-  if (shape < kNumTiles) {
-    const TileLaunch big = t;
-    tile_kernel(dtype, true, shape, t);
-    if (!tile_addresses(t.tm, p.lda, p.ldsa) ||
-        ((p.M + (E < p.M ? E : p.M) * (t.tm - 1)) / t.tm) * ((p.N + t.tn - 1) / t.tn) > INT32_MAX)
-      t = big;
-  }
   // Upper bound of the experts' m-tiles: sum ceil(M_e / tm) over at most
   // min(E, T) experts that have rows.
   const long long rows_e = E < p.M ? E : p.M;
+  const TileProblem problem{tile_family(dtype), p.M, p.N, p.ns,
+                            ((double)p.M + (double)rows_e * p.N) * p.K * value_bytes(dtype) + 2.0 * p.M * p.N,
+                            p.lda, p.ldsa, cus};
+  const int shape = pick_moe_tile(problem, E);
+  if (shape < kNumTiles) tile_kernel(dtype, true, shape, t);
   const long long tiles_m = ((long long)p.M + rows_e * (t.tm - 1)) / t.tm;
   p.tiles_n = (p.N + t.tn - 1) / t.tn;
   if (tiles_m * p.tiles_n > INT32_MAX) return G9_ERR_SHAPE;

@@ -2,6 +2,8 @@
 // (g9_tile.hpp) or the 256x256 kernels' tile.  Host code only.
 #pragma once
 
+#include <climits>
+
 namespace g9 {
 
 struct GemmParams;
@@ -30,9 +32,13 @@ inline bool tile_addresses(int tm, long long lda, long long ldsa) {
 // Cost of one tile in microseconds, fixed + per K stage (128 bytes of a row),
 // by operand size (16-bit, BF8, MXFP4): the least-squares fit (in the
 // logarithm) of predict() to the kernels' times on 43 shapes from 1 x 1024 to
-// 8192 x 512 and 5000 x 4096, K 512-14336, one MI355X (256 CUs).  Over those
-// shapes and the three types the tile picked takes 0.2% longer than the
-// fastest one on average, 10% at most.
+// 8192 x 512 and 5000 x 4096, K 512-14336, one MI355X (256 CUs), operands in
+// the 256 MB memory-side cache.  Over those shapes and the three types the tile
+// picked takes 0.2% longer than the fastest one on average, 10% at most; they
+// are the shapes of the fit.  Rows that are no whole number of 128-byte lines
+// apart take the small tiles up to twice as long as predicted, but of 240
+// drawn data-parallel calls with such rows (up to 600 256x256 tiles) none took
+// more than 3% longer than on 256x256 tiles.
 struct TileCost {
   float fixed, stage;
 };
@@ -46,46 +52,97 @@ constexpr TileCost kTileCost[3][kNumTiles + 1] = {
 
 // Predicted time (us) of `tiles` tiles of shape index `shape` over `ns` K
 // stages on `cus` CUs, `bytes` the operands and outputs: whole rounds of one
-// tile per CU, against reading the operands at 5.2 TB/s; a quarter of the
-// smaller of the two does not overlap.
-inline double tile_time(int family, int shape, double tiles, int ns, double bytes, int cus) {
+// tile per CU (their time times `slow`), against reading the operands at
+// 5.2 TB/s; a quarter of the smaller of the two does not overlap.
+inline double tile_time(int family, int shape, double tiles, int ns, double bytes, int cus, double slow = 1.0) {
   const TileCost& c = kTileCost[family][shape];
   const double rounds = (double)(long long)((tiles + cus - 1) / cus);
-  const double x = (c.fixed + ns * (double)c.stage) * (rounds < 1 ? 1 : rounds), y = 1.0 + bytes * (1.0 / 5.2e6);
+  const double x = slow * (c.fixed + ns * (double)c.stage) * (rounds < 1 ? 1 : rounds), y = 1.0 + bytes * (1.0 / 5.2e6);
   return 2.5 + (x > y ? x + 0.25 * y : y + 0.25 * x);
 }
 
-// Shape index with the smallest predicted time for an M x N output.  The
-// 256x256 tile (kNumTiles) is preferred within 7%: its many-round times, where
-// the chip is power-limited, are the model's least accurate ones.
-inline int pick_tile(int family, long long M, long long N, int ns, double bytes, int cus, double* time = nullptr) {
+// What the choice depends on: an M x N output of operand size `family`, `ns` K
+// stages, `bytes` of operands and output, A rows (and row-major A scales) lda
+// (ldsa) bytes apart, on `cus` CUs.
+struct TileProblem {
+  int family;
+  long long M, N;
+  int ns;
+  double bytes;
+  long long lda, ldsa;
+  int cus;
+};
+
+inline double tile_count(long long M, long long N, int shape) {
+  return (double)((M + kTileShapes[shape][0] - 1) / kTileShapes[shape][0]) *
+         (double)((N + kTileShapes[shape][1] - 1) / kTileShapes[shape][1]);
+}
+
+// Shape index with the smallest predicted time among the tiles that can
+// address the operands.  The 256x256 tile (kNumTiles) is preferred within 7%:
+// its many-round times, where the chip is power-limited, are the model's least
+// accurate ones.
+inline int pick_tile(const TileProblem& p) {
   int best = kNumTiles;
   double best_t = 0;
   for (int i = kNumTiles; i >= 0; --i) {
-    const double tiles = (double)((M + kTileShapes[i][0] - 1) / kTileShapes[i][0]) *
-                         (double)((N + kTileShapes[i][1] - 1) / kTileShapes[i][1]);
-    const double t = tile_time(family, i, tiles, ns, bytes, cus) * (i == kNumTiles ? 0.93 : 1.0);
+    const double tiles = tile_count(p.M, p.N, i);
+    if (i < kNumTiles && (tiles > INT_MAX || !tile_addresses(kTileShapes[i][0], p.lda, p.ldsa))) continue;
+    const double t = tile_time(p.family, i, tiles, p.ns, p.bytes, p.cus) * (i == kNumTiles ? 0.93 : 1.0);
     if (i == kNumTiles || t < best_t) {
       best = i;
       best_t = t;
     }
   }
-  if (time) *time = best_t;
   return best;
 }
 
-// The same for a grouped GEMM of T rows over E experts.  The rows per expert
-// are on the device: an expert is taken to have the average of the experts
-// that can have rows, and half an m-tile more than its rows fill.
-inline int pick_moe_tile(int family, long long T, long long E, long long N, int ns, double row_bytes, int cus) {
-  const double experts = (double)(E < T ? E : T), rows = T / experts;
-  const double bytes = (T + experts * N) * row_bytes + 2.0 * T * N;
+// Predicted time (us) of split-K with S segments for each of `tiles` 256x256
+// tiles: launches and a tile's fixed cost, a segment's stages (`ragged`: rows
+// that are no whole number of 128-byte lines apart), and a share per 256 KiB
+// partial of the reduction.  Least-squares fit to the split's times on 231
+// drawn shapes near the rule below (rms error 7%).
+constexpr float kSplitStage[3] = {1.16f, 1.12f, 1.35f};
+inline double splitk_time(int family, int ns, long long tiles, int S, bool ragged) {
+  return 13.1 + kSplitStage[family] * (ragged ? 1.12 : 1.0) * ((ns + S - 1) / S) + 0.0515 * (double)(tiles * S);
+}
+
+// Whether a split-K call runs data-parallel on small tile `shape` instead.
+// The tiles' times depend on where the operands are: as predicted in the
+// memory-side cache, 1.2 to 1.5 times that from HBM, where the split's, on
+// tiles that read each operand less often, grow by 1 to 5%.  A launch cannot
+// know, so the factors take the smallest geometric mean of both over the 231
+// shapes (0.3% above the better of the two on average): FP16/BF16 tiles, whose
+// predictions are up to 15% high, within 1.05 of the split, BF8 and MXFP4
+// below 0.88, and rows off 128-byte lines, which cost the tiles up to twice
+// their prediction, below 0.7.  Operands of more than 140 MB do not stay in
+// the cache from one call to the next.  None of the 231 then loses to the
+// split with its operands in the cache; with 1.0, 1.0 and 0.65 in their place
+// 13 did, by up to 1.5 times (BF8 7972 x 896 x 22272: 159 against 122 us).
+inline bool tile_beats_split(const TileProblem& p, int shape, long long tiles, int S, bool ragged) {
+  if (shape >= kNumTiles) return false;
+  const double slow = p.bytes > 140e6 ? 1.3 : 1.0;
+  const double t = tile_time(p.family, shape, tile_count(p.M, p.N, shape), p.ns, p.bytes, p.cus, slow);
+  return t < (ragged ? 0.7 : p.family == 0 ? 1.05 : 0.88) * splitk_time(p.family, p.ns, tiles, S, ragged);
+}
+
+// The choice for a grouped GEMM of p.M rows over E experts.  The rows per
+// expert are on the device: an expert is taken to have the average of the
+// experts that can have rows, and half an m-tile more than its rows fill.
+inline int pick_moe_tile(const TileProblem& p, long long E) {
+  const long long rows_e = E < p.M ? E : p.M;
+  const double experts = (double)rows_e, rows = p.M / experts;
   int best = kNumTiles;
   double best_t = 0;
   for (int i = kNumTiles; i >= 0; --i) {
-    const double per = rows / kTileShapes[i][0] + 0.5;
-    const double tiles = experts * (per < 1 ? 1 : per) * (double)((N + kTileShapes[i][1] - 1) / kTileShapes[i][1]);
-    const double t = tile_time(family, i, tiles, ns, bytes, cus) * (i == kNumTiles ? 0.93 : 1.0);
+    const int tm = kTileShapes[i][0];
+    const long long tn = (p.N + kTileShapes[i][1] - 1) / kTileShapes[i][1];
+    // The grid's bound (launch_moe) has to be a 32-bit number.
+    if (i < kNumTiles && ((double)((p.M + rows_e * (tm - 1)) / tm) * tn > INT_MAX || !tile_addresses(tm, p.lda, p.ldsa)))
+      continue;
+    const double per = rows / tm + 0.5;
+    const double tiles = experts * (per < 1 ? 1 : per) * (double)tn;
+    const double t = tile_time(p.family, i, tiles, p.ns, p.bytes, p.cus) * (i == kNumTiles ? 0.93 : 1.0);
     if (i == kNumTiles || t < best_t) {
       best = i;
       best_t = t;
