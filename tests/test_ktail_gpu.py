@@ -14,6 +14,7 @@ import numpy as np
 import pytest
 import torch
 
+import launched
 from gfx950_gluon_tutorials_amd.gemm import _launch
 from oracle import gemm_ref as R
 
@@ -115,6 +116,36 @@ def test_a16w16_k_tail_random_and_streamk_bitwise(gpu, waves):
     got = c_dp.float().cpu().numpy()[rows]
     atol = 1e-2 * np.sqrt(K) * 0.01
     assert np.allclose(got, want, rtol=1e-2, atol=atol), np.abs(got - want).max()
+
+
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("dtype,M,N,K,splits", [("f16", 360, 1385, 6240, 14), ("bf16", 1443, 178, 7448, 15),
+                                                ("bf8", 207, 1209, 16608, 15), ("bf8", 198, 2148, 11616, 13)])
+def test_split_k_tails_exact(gpu, dtype, M, N, K, splits, waves):
+    """The shapes above run on small tiles under "splitk"; these split, the first segment with the partial stage."""
+    _say(f"split {dtype} {M}x{N}x{K} {waves}w")
+    g = np.random.default_rng(6)
+    if dtype == "bf8":
+        codes = np.array([0xBC, 0x00, 0x3C], dtype=np.uint8)  # e5m2 -1.0, 0, 1.0
+        a, b = codes[g.integers(0, 3, size=(M, K))], codes[g.integers(0, 3, size=(N, K))]
+        av = _poisoned(a, torch.float8_e5m2, gpu, nan_code=0x7F)
+        bv = _poisoned(b, torch.float8_e5m2, gpu, nan_code=0x7F)
+        c = torch.empty(M, N, dtype=torch.bfloat16, device=gpu)
+        launched.a8w8(splits, av, bv.T, c, schedule="splitk", waves=waves)
+        _launch.gemm_a8w8(av, bv.T, c, schedule="splitk", waves=waves)
+        want = R.a8w8_ref(a, b, out_dtype="bf16")
+    else:
+        tdt = torch.float16 if dtype == "f16" else torch.bfloat16
+        a, b = _small_ints(g, (M, K)), _small_ints(g, (N, K))
+        av, bv = _poisoned(a, tdt, gpu), _poisoned(b, tdt, gpu)
+        c = torch.empty(M, N, dtype=tdt, device=gpu)
+        launched.a16w16(splits, av, bv.T, c, schedule="splitk", waves=waves)
+        _launch.gemm_a16w16(av, bv.T, c, schedule="splitk", waves=waves)
+        want = R.a16w16_ref(a, b, dtype)
+    torch.cuda.synchronize()
+    got = c.float().cpu().numpy()
+    assert np.isfinite(got).all(), "a masked chunk was loaded"
+    np.testing.assert_array_equal(got, want.astype(np.float32))
 
 
 def test_k_granularity_is_still_enforced(gpu):

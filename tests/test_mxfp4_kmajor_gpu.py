@@ -21,6 +21,7 @@ import numpy as np
 import pytest
 import torch
 
+import launched
 from gfx950_gluon_tutorials_amd import _lib, quant
 from gfx950_gluon_tutorials_amd.gemm import _launch
 from gfx950_gluon_tutorials_amd.gemm.intra_wave.a4w4 import matmul as a4w4_matmul
@@ -125,29 +126,31 @@ def test_stage_counts_and_ragged_edges(gpu, ns):
 
 @pytest.mark.parametrize("schedule", ["dp", "streamk", "splitk"])
 @pytest.mark.parametrize("M,N,K", [(3, 9, 1024), (37, 50, 512), (129, 255, 768), (301, 267, 2304), (517, 1798, 1536),
-                                   (1671, 1165, 1536), (4099, 4093, 768)])
+                                   (1671, 1165, 1536), (4099, 4093, 768), (1163, 837, 20224)])
 def test_row_counts_off_dwords(gpu, M, N, K, schedule):
     """Row counts that are no multiple of 4: the last group's last rows share a
     dword with padding.  Bit-equal to the row-major scales on small and 256x256
     tiles, whole and split."""
     _say(f"a4w4 K-major, rows off dwords {M}x{N}x{K} {schedule}")
     gen = torch.Generator().manual_seed(M + N)
-    pa, sa = (t.to(gpu) for t in quant.quantize_mxfp4(torch.randn(M, K, generator=gen)))
-    pb, sb = (t.to(gpu) for t in quant.quantize_mxfp4(torch.randn(N, K, generator=gen)))
+    pa, sa = quant.quantize_mxfp4(torch.randn(M, K, generator=gen).to(gpu))
+    pb, sb = quant.quantize_mxfp4(torch.randn(N, K, generator=gen).to(gpu))
+    if K == 20224 and schedule == "splitk":  # the other split-K calls run on small tiles or unsplit
+        launched.a4w4(10, pa, pb, sa, sb, torch.empty(M, N, dtype=torch.bfloat16, device=gpu), schedule=schedule)
     rm = _run(gpu, pa, pb, sa, sb, schedule=schedule)
     km = _run(gpu, pa, pb, _kmajor(sa, pad_rows=-M % 4), _kmajor(sb, pad_rows=4 + -N % 4), schedule=schedule)
     torch.cuda.synchronize()
     np.testing.assert_array_equal(_bits(km), _bits(rm))
 
 
-@pytest.mark.parametrize("M,N,K", [(3840, 3840, 4096), (1280, 2304, 2560)])
+@pytest.mark.parametrize("M,N,K", [(3840, 3840, 4096), (1280, 2304, 2560), (1160, 835, 20224)])
 def test_streamk_and_splitk(gpu, M, N, K):
     _say(f"a4w4 K-major stream-K / split-K {M}x{N}x{K}")
     gen = torch.Generator().manual_seed(M + K)
     pa, sa = quant.quantize_mxfp4(torch.randn(M, K, generator=gen))
     pb, sb = quant.quantize_mxfp4(torch.randn(N, K, generator=gen))
     a, b = pa.to(gpu), pb.to(gpu)
-    ka, kb = _kmajor(sa.to(gpu), pad_rows=4), _kmajor(sb.to(gpu))
+    ka, kb = _kmajor(sa.to(gpu), pad_rows=4), _kmajor(sb.to(gpu), pad_rows=-N % 4)
     dp = _run(gpu, a, b, ka, kb)
     sk = _run(gpu, a, b, ka, kb, schedule="streamk")
     sp = _run(gpu, a, b, ka, kb, schedule="splitk")
@@ -155,6 +158,8 @@ def test_streamk_and_splitk(gpu, M, N, K):
     torch.cuda.synchronize()
     assert torch.equal(sk, dp)
     assert torch.equal(sp, rm_sp)
+    if (M, N, K) == (1160, 835, 20224):
+        launched.a4w4(10, a, b, ka, kb, torch.empty_like(sp), schedule="splitk")
     rows = torch.from_numpy(np.unique(np.r_[0, M - 1, np.random.default_rng(3).integers(0, M, 64)]))
     ref = R.a4w4_ref(pa[rows].numpy(), pb.numpy(), sa[rows].numpy(), sb.numpy(), "bf16")
     assert R.rel_frobenius(sp[rows].float().cpu().numpy(), ref) <= 1e-3

@@ -15,6 +15,7 @@ import numpy as np
 import pytest
 import torch
 
+import launched
 from gfx950_gluon_tutorials_amd import _lib, quant
 from gfx950_gluon_tutorials_amd.gemm import _launch
 from gfx950_gluon_tutorials_amd.gemm.prepared import PreparedGemm
@@ -43,11 +44,13 @@ def _f16_sets(gpu, M, N, K, dtype, n, seed):
 @pytest.mark.parametrize("schedule,waves,M,N,K", [
     ("dp", 4, 1000, 700, 1032), ("dp", 8, 600, 520, 2048), ("streamk", 4, 1300, 1100, 2048),
     ("streamk", 8, 1024, 768, 4096), ("streamk_half", 4, 600, 900, 1536), ("splitk", 4, 512, 1024, 4096),
-    ("splitk", 8, 256, 512, 2048)])
+    ("splitk", 8, 256, 512, 2048), ("splitk", 4, 512, 1024, 8200), ("splitk", 8, 1388, 741, 7040)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_a16w16_slots_match_the_wrapper(gpu, schedule, waves, M, N, K, dtype):
     _say(f"prepared a16w16 {schedule} {waves}w {M}x{N}x{K} {dtype}")
     sets = _f16_sets(gpu, M, N, K, dtype, 3, M + N + K)
+    if schedule == "splitk":  # the first two run on small tiles, the others split
+        launched.a16w16({4096: "64x32", 2048: "16x32", 8200: 15, 7040: 11}[K], *sets[0], schedule=schedule, waves=waves)
     prep = PreparedGemm.a16w16(sets, schedule=schedule, waves=waves)
     assert prep.slots == 3
     ref = [_launch.gemm_a16w16(a, b, torch.empty_like(c), schedule=schedule, waves=waves) for a, b, c in sets]
@@ -61,7 +64,7 @@ def test_a16w16_slots_match_the_wrapper(gpu, schedule, waves, M, N, K, dtype):
 
 @pytest.mark.parametrize("schedule,waves", [("dp", 4), ("dp", 8), ("streamk", 4), ("splitk", 4)])
 def test_a8w8_slots_match_the_wrapper(gpu, schedule, waves):
-    M, N, K = (512, 1024, 4096) if schedule == "splitk" else (900, 1300, 2048)
+    M, N, K = (207, 1209, 16608) if schedule == "splitk" else (900, 1300, 2048)
     _say(f"prepared a8w8 {schedule} {waves}w {M}x{N}x{K}")
     gen = torch.Generator().manual_seed(7)
     sets = []
@@ -69,6 +72,8 @@ def test_a8w8_slots_match_the_wrapper(gpu, schedule, waves):
         qa, sa = quant.quantize_e5m2(torch.randn(M, K, generator=gen).to(gpu))
         qb, sb = quant.quantize_e5m2(torch.randn(N, K, generator=gen).to(gpu))
         sets.append((qa, qb.T, torch.empty(M, N, dtype=torch.bfloat16, device=gpu), sa, sb))
+    if schedule == "splitk":
+        launched.a8w8(15, *sets[0], schedule=schedule, waves=waves)
     prep = PreparedGemm.a8w8(sets, schedule=schedule, waves=waves)
     ref = [_launch.gemm_a8w8(a, b, torch.empty_like(c), a_scale=sa, b_scale=sb, schedule=schedule, waves=waves)
            for a, b, c, sa, sb in sets]
@@ -84,13 +89,13 @@ def test_a8w8_slots_match_the_wrapper(gpu, schedule, waves):
     ("row", "dp", 4), ("row", "dp", 8), ("row", "streamk", 4), ("row", "splitk", 4), ("kmajor", "dp", 4),
     ("kmajor", "streamk", 4), ("preshuffled", "dp", 4)])
 def test_a4w4_slots_match_the_wrapper(gpu, layout, schedule, waves):
-    M, N, K = (512, 1024, 4096) if schedule == "splitk" else (1024, 768, 2048)
+    M, N, K = (457, 2478, 20736) if schedule == "splitk" else (1024, 768, 2048)
     _say(f"prepared a4w4 {layout} {schedule} {waves}w {M}x{N}x{K}")
     gen = torch.Generator().manual_seed(11)
     sets = []
     for _ in range(2):
-        pa, sa = quant.quantize_mxfp4(torch.randn(M, K, generator=gen))
-        pb, sb = quant.quantize_mxfp4(torch.randn(N, K, generator=gen))
+        pa, sa = quant.quantize_mxfp4(torch.randn(M, K, generator=gen).to(gpu))
+        pb, sb = quant.quantize_mxfp4(torch.randn(N, K, generator=gen).to(gpu))
         if layout == "kmajor":
             sa, sb = sa.t().contiguous().t(), sb.t().contiguous().t()
         elif layout == "preshuffled":
@@ -99,6 +104,8 @@ def test_a4w4_slots_match_the_wrapper(gpu, layout, schedule, waves):
                      torch.empty(M, N, dtype=torch.bfloat16, device=gpu)))
     if layout == "kmajor":
         assert sets[0][2].stride(0) == 1  # the views survived the copy to the device
+    if schedule == "splitk":
+        launched.a4w4(9, *sets[0], schedule=schedule, waves=waves)
     prep = PreparedGemm.a4w4(sets, schedule=schedule, waves=waves)
     ref = [_launch.gemm_a4w4(a, b, sa, sb, torch.empty_like(c), schedule=schedule, waves=waves)
            for a, b, sa, sb, c in sets]
@@ -177,7 +184,7 @@ def test_c_abi_plan_is_plain_data(gpu):
     np.testing.assert_array_equal(_bits(c), _bits(c_ref))
 
 
-@pytest.mark.parametrize("schedule,M,N,K", [("dp", 1000, 700, 2048), ("splitk", 512, 1024, 4096),
+@pytest.mark.parametrize("schedule,M,N,K", [("dp", 1000, 700, 2048), ("splitk", 512, 1024, 8200),
                                             ("streamk", 1300, 1100, 2048), ("streamk_half", 600, 900, 1536)])
 def test_prepared_launches_replay_in_a_graph(gpu, schedule, M, N, K):
     """Two slots' launches captured in one HIP graph (a plan launch is a bare
@@ -188,6 +195,8 @@ def test_prepared_launches_replay_in_a_graph(gpu, schedule, M, N, K):
     owner clears its flag, so each replay starts from clear flags."""
     _say(f"prepared {schedule} {M}x{N}x{K} captured in a graph")
     sets = _f16_sets(gpu, M, N, K, torch.float16, 2, 99)
+    if schedule == "splitk":
+        launched.a16w16(15, *sets[0], schedule=schedule)
     want = [_launch.gemm_a16w16(a, b, torch.empty_like(c), schedule=schedule) for a, b, c in sets]
     torch.cuda.synchronize()
     side = torch.cuda.Stream(device=gpu)

@@ -5,8 +5,8 @@ types, of 256 for MXFP4) from a fixed seed and checks the invariants the
 schedules promise on the same inputs:
 
 * FP16: stream-K with 256x256 and with 256x128 tiles bit-identical to
-  data-parallel, split-K within the FP16 tolerance of it, 8 waves
-  bit-identical to 4 waves;
+  data-parallel, split-K (which takes small tiles on shapes of this size)
+  within the FP16 tolerance of it, 8 waves bit-identical to 4 waves;
 * MXFP4: K-major and preshuffled scale layouts bit-identical to row-major,
   stream-K bit-identical to data-parallel.
 

@@ -14,6 +14,7 @@ stream-K launches of different tile counts.
 import pytest
 import torch
 
+import launched
 from gfx950_gluon_tutorials_amd.gemm import _launch
 
 pytestmark = pytest.mark.gpu
@@ -32,13 +33,15 @@ def _operands(gen, M, N, K, dev):
 def test_streamk_and_splitk_on_two_streams_at_once(gpu):
     g = torch.Generator().manual_seed(61)
     # 272 tiles: stream-K hands partial tiles along K chains (flags in use);
-    # 512 x 4096: split-K runs 8 segments per tile (partials in use).
+    # 512 x 4096 x 8200: split-K runs 8 segments per tile (partials in use).
     sk_shape = (4352, 4096, 2048)
-    sp_shape = (512, 4096, 8192)
+    sp_shape = (512, 4096, 8200)
     sk_in = [_operands(g, *sk_shape, gpu) for _ in range(2)]
     sp_in = [_operands(g, *sp_shape, gpu) for _ in range(2)]
     _say("single-stream references: data-parallel for stream-K, split-K alone")
     want_sk, want_sp = [], []
+    launched.a16w16(8, sp_in[0][0], sp_in[0][1].T, torch.empty(sp_shape[0], sp_shape[1], dtype=torch.float16, device=gpu),
+                    schedule="splitk")
     for (a, b), (x, y) in zip(sk_in, sp_in):
         want_sk.append(_launch.gemm_a16w16(a, b.T, torch.empty(sk_shape[0], sk_shape[1], dtype=torch.float16,
                                                                  device=gpu), schedule="dp"))
