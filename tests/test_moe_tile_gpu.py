@@ -1,6 +1,8 @@
-"""Grouped GEMMs on the small output tiles (few rows per expert): each expert's
-rows equal, bit for bit, stream-K's on that expert's slice (256x256 tiles, the
-same MFMA sequence); rows past the last expert's stay as they were.
+"""Grouped GEMMs on every output tile, 16x16 to 256x256: each expert's rows equal,
+bit for bit, stream-K's on that expert's slice (256x256 tiles, the same MFMA
+sequence); rows past the last expert's stay as they were.  Each shape names the
+tile that the launch picks there (256 CUs), and has experts of more than one
+tile's rows and a last column tile that is not full.
 
 E past 64 takes the expert lookup through more than one pass; empty experts,
 one-row experts and experts just past a tile's rows are in every table."""
@@ -9,6 +11,7 @@ import numpy as np
 import pytest
 import torch
 
+import tile_pick
 from gfx950_gluon_tutorials_amd import quant
 from gfx950_gluon_tutorials_amd.gemm import _launch
 from gfx950_gluon_tutorials_amd.gemm.moe import moe_matmul, moe_matmul_a4w4, moe_matmul_a8w8
@@ -23,13 +26,30 @@ def _counts(E, mean, seed):
     return c
 
 
-@pytest.mark.parametrize("kind", ["f16", "bf16", "bf8", "mxfp4"])
-@pytest.mark.parametrize("E,mean,N,K", [(70, 3, 136, 512), (9, 17, 1032, 2048), (130, 40, 264, 768), (6, 150, 520, 1024)])
-def test_moe_tile_bits(gpu, kind, E, mean, N, K):
+# (E, mean rows, N, K, tile)
+ALL = [(70, 3, 136, 512, "64x64"), (9, 17, 1032, 2048, "64x64"), (130, 40, 264, 768, "64x64"),
+       (6, 150, 520, 1024, "64x64")]
+SHAPES16 = [(3, 16, 24, 512, "16x16"), (4, 86, 360, 512, "16x32"), (6, 79, 304, 576, "32x32"), (4, 33, 56, 320, "64x32"),
+            (5, 154, 824, 256, "64x64"), (4, 378, 984, 768, "128x64"), (5, 209, 3144, 256, "128x128"),
+            (66, 230, 520, 512, "128x128"), (6, 909, 1296, 256, "256x128"), (12, 462, 1656, 256, "256x256"),
+            (66, 230, 1032, 256, "256x256")]
+SHAPES8 = [(4, 8, 56, 512, "16x16"), (4, 86, 296, 1152, "16x32"), (4, 49, 432, 512, "32x32"), (5, 115, 592, 512, "64x32"),
+           (4, 169, 1008, 512, "64x64"), (6, 361, 520, 1408, "128x64"), (5, 389, 2200, 512, "128x128"),
+           (9, 534, 1264, 512, "256x128"), (6, 1017, 1720, 512, "256x256")]
+SHAPES4 = [(4, 22, 24, 1024, "16x16"), (4, 111, 248, 2048, "16x32"), (3, 78, 664, 1024, "32x32"),
+           (6, 61, 680, 1024, "64x32"), (5, 168, 688, 1280, "64x64"), (4, 426, 792, 1792, "128x64"),
+           (4, 819, 792, 1280, "128x128"), (6, 470, 2280, 1024, "256x128"), (9, 284, 2968, 1024, "256x256")]
+CASES = [(kind, *s) for kind, shapes in (("f16", SHAPES16), ("bf16", SHAPES16), ("bf8", SHAPES8), ("mxfp4", SHAPES4))
+         for s in ALL + shapes]
+
+
+@pytest.mark.parametrize("kind,E,mean,N,K,tile", CASES)
+def test_moe_tile_bits(gpu, kind, E, mean, N, K, tile):
     counts = _counts(E, mean, E + N)
     off = np.concatenate([[0], np.cumsum(counts)])
     T = int(off[-1]) + 5  # rows no expert owns
-    print(f"\n[case] moe {kind} E={E} T={T} N={N} K={K}", flush=True)
+    print(f"\n[case] moe {kind} E={E} T={T} N={N} K={K} {tile}", flush=True)
+    assert tile_pick.moe(kind, T, E, N, K) == tile
     g = torch.Generator(device=gpu).manual_seed(E)
     offs = torch.tensor(off, dtype=torch.int32, device=gpu)
     x = torch.randn(T, K, generator=g, device=gpu)

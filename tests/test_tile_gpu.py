@@ -11,6 +11,8 @@ slice of a wider buffer, whose padding must survive.
 import pytest
 import torch
 
+import launched
+import tile_pick
 from gfx950_gluon_tutorials_amd import quant
 from gfx950_gluon_tutorials_amd.gemm import _launch
 
@@ -49,23 +51,26 @@ def test_a16w16_tile_bits(gpu, tile, dtype, waves):
     a = torch.randn(M, K, generator=g, device=gpu).to(dtype)
     b = torch.randn(N, K, generator=g, device=gpu).to(dtype)
     buf, c = _out(gpu, M, N, dtype)
+    launched.a16w16(tile, a, b.T, c, waves=waves)
     _launch.gemm_a16w16(a, b.T, c, waves=waves)
     want = _launch.gemm_a16w16(a, b.T, torch.empty(M, N, dtype=dtype, device=gpu), schedule="streamk", waves=waves)
     _same(buf, c, want)
 
 
+@pytest.mark.parametrize("waves", [4, 8])
 @pytest.mark.parametrize("out", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("tile", TILES)
-def test_a8w8_tile_bits(gpu, tile, out):
+def test_a8w8_tile_bits(gpu, tile, out, waves):
     M, N, K = SHAPES8[tile]
-    print(f"\n[case] a8w8 {tile} {M}x{N}x{K} {out}", flush=True)
+    print(f"\n[case] a8w8 {tile} {M}x{N}x{K} {out} {waves}w", flush=True)
     g = torch.Generator(device=gpu).manual_seed(M + N)
     a, sa = quant.quantize_e5m2(torch.randn(M, K, generator=g, device=gpu))
     b, sb = quant.quantize_e5m2(torch.randn(N, K, generator=g, device=gpu))
     buf, c = _out(gpu, M, N, out)
-    _launch.gemm_a8w8(a, b.T, c, a_scale=sa, b_scale=sb)
+    launched.a8w8(tile, a, b.T, c, waves=waves)
+    _launch.gemm_a8w8(a, b.T, c, a_scale=sa, b_scale=sb, waves=waves)
     want = _launch.gemm_a8w8(a, b.T, torch.empty(M, N, dtype=out, device=gpu), a_scale=sa, b_scale=sb,
-                             schedule="streamk")
+                             schedule="streamk", waves=waves)
     _same(buf, c, want)
 
 
@@ -79,8 +84,8 @@ def _k_major(s):
 @pytest.mark.parametrize("tile", TILES)
 def test_a4w4_tile_bits(gpu, tile, layout):
     M, N, K = SHAPES4[tile]
-    if layout == "kmajor":  # whole dwords of rows in each scale group
-        M, N = M + 4 - M % 4, N + 4 - N % 4
+    if layout == "kmajor":  # the last group's rows end inside a dword, for A and for B
+        M, N = M | 1, N | 3
     print(f"\n[case] a4w4 {tile} {M}x{N}x{K} {layout}", flush=True)
     g = torch.Generator(device=gpu).manual_seed(M + N)
     a, sa = quant.quantize_mxfp4(torch.randn(M, K, generator=g, device=gpu))
@@ -91,6 +96,7 @@ def test_a4w4_tile_bits(gpu, tile, layout):
     elif layout == "preshuffled":
         sa, sb = quant.preshuffle_e8m0(sa), quant.preshuffle_e8m0(sb)
     buf, c = _out(gpu, M, N, torch.bfloat16)
+    launched.a4w4(tile, a, b, sa, sb, c)
     _launch.gemm_a4w4(a, b, sa, sb, c)
     _same(buf, c, want)
 
@@ -115,6 +121,10 @@ def test_wide_rows(gpu, op, stride):
     if stride == 2**24 and not op.startswith("mxfp4"):
         K = 1024
     print(f"\n[case] wide rows {op} {M}x{N}x{K} stride {stride}", flush=True)
+    kind = op.split("_")[0]
+    assert tile_pick.dense(kind, M, N, K) == "256x128"
+    if op != "mxfp4_scales":
+        assert (tile_pick.dense(kind, M, N, K, lda=stride) == "256x128") == (stride < 2**23)
     g = torch.Generator(device=gpu).manual_seed(K)
     a = torch.randn(M, K, generator=g, device=gpu)
     b = torch.randn(N, K, generator=g, device=gpu)
