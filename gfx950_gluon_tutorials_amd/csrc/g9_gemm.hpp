@@ -736,8 +736,13 @@ struct Pipe {
       } else {
         // Row-major scales: lane l of part j fetches the 16-byte half of row
         // 32 j + l / 2 that belongs in its LDS half under the bit-3 row swap.
+        // A chunk can reach past a row's K/32 = 8 ns bytes; the range ends with
+        // those of the last row, behind which the array need not go on (as a
+        // scalar: without the readfirstlane the loop's DMAs rebuild the
+        // resource from VGPRs, 4096 x 4096 x 8192 58.1 -> 59.1 us).
         const unsigned char* hbase = (sa ? p.a_sc : p.b_sc) + (size_t)hrow * lds;
-        rS = make_rsrc(hbase, (u32)hvalid * lds);
+        const u32 end = hvalid ? (u32)(hvalid - 1) * lds + 8u * (u32)p.ns : 0u;
+        rS = make_rsrc(hbase, (u32)__builtin_amdgcn_readfirstlane((int)end));
 #pragma unroll
         for (int j = 0; j < SP; ++j) {
           const int row = r0 + 32 * j + (lane >> 1);

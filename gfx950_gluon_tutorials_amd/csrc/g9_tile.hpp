@@ -178,8 +178,10 @@ struct TilePipe {
           vs[k] = grp < 32 ? (u32)grp * ld + 16u * part : kDeadOff;
           cstep[k] = 32u * ld;
         } else {
-          // Row m of the chunk: 32 bytes at m * ld + 32 c.
-          rs[k] = make_rsrc(base + (size_t)row0 * ld, rows * ld);
+          // Row m of the chunk: 32 bytes at m * ld + 32 c, up to the last
+          // row's last byte and kept scalar, as in the 256x256 kernels.
+          const u32 end = rows ? (rows - 1) * ld + 8u * (u32)p.ns : 0u;
+          rs[k] = make_rsrc(base + (size_t)row0 * ld, (u32)__builtin_amdgcn_readfirstlane((int)end));
           vs[k] = (u32)(32 * unit + (lane >> 1)) * ld + 16u * (lane & 1);
           cstep[k] = kScRowBytes;
         }

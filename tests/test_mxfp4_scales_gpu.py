@@ -4,6 +4,7 @@
   row-major-scale kernel on the same values (same data, MFMAs and order), at
   the BASELINE MXFP4 configuration and on ragged shapes of 1-17 stages (chunks
   cut short by K), and within the oracle's tolerance.
+* Row-major scales in a column slice of a wider array: bit-identical to packed ones.
 * Extreme E8M0 codes (0-8 and 246-254: operands that are fp32 subnormals or
   near fp32's top when dequantized): with one operand's scales small and the
   other's large every product is a normal fp32 value and the oracle's result is
@@ -106,6 +107,31 @@ def test_preshuffled_scales_with_padded_chunk_stride(gpu):
     want = _launch.gemm_a4w4(a, b, sa.to(gpu), sb.to(gpu), torch.empty(M, N, dtype=torch.float16, device=gpu))
     torch.cuda.synchronize()
     assert torch.equal(c, want)
+
+
+def _last_columns(s, ld):
+    """The scales as the last columns of rows `ld` bytes apart: the last row ends the storage."""
+    wide = torch.full((s.shape[0], ld), 255, dtype=torch.uint8, device=s.device)  # NaN scales outside the view
+    v = wide[:, ld - s.shape[1]:]
+    v.copy_(s)
+    return v
+
+
+@pytest.mark.parametrize("schedule,waves", [("dp", 4), ("dp", 8), ("streamk", 4), ("streamk", 8), ("splitk", 4),
+                                            ("splitk", 8)])
+@pytest.mark.parametrize("M,N,K", [(3, 9, 256), (129, 257, 1280), (517, 1798, 1536), (4099, 4093, 768)])
+def test_row_major_scales_of_a_wider_array(gpu, M, N, K, schedule, waves):
+    """A column slice of a scale array, read in place: bit-equal to the packed scales."""
+    _say(f"a4w4 sliced row-major scales {M}x{N}x{K} {schedule} {waves}w")
+    gen = torch.Generator(device=gpu).manual_seed(M + N)
+    pa, sa = quant.quantize_mxfp4(torch.randn(M, K, generator=gen, device=gpu))
+    pb, sb = quant.quantize_mxfp4(torch.randn(N, K, generator=gen, device=gpu))
+    va, vb = _last_columns(sa, K // 32 + 4), _last_columns(sb, K // 32 + 24)
+    assert _launch._scales_ok(va) and _launch._scales_ok(vb)
+    c = [_launch.gemm_a4w4(pa, pb, x, y, torch.empty(M, N, dtype=torch.bfloat16, device=gpu), schedule=schedule,
+                           waves=waves) for x, y in ((va, vb), (sa, sb))]
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(_bits(c[0]), _bits(c[1]))
 
 
 def _extreme_case(gen, M, N, K, a_codes, b_codes):

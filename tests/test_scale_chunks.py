@@ -287,3 +287,20 @@ def test_k_major_ranges_hold_every_valid_row_and_stay_inside_the_array(half):
                 assert end == 0 or base + end <= groups * ld
                 last = (groups - 1) * ld + valid - 1
                 assert valid == 0 or last // 4 * 4 + 4 <= end
+
+
+@pytest.mark.parametrize("half", [128, 16, 32, 64, 256])
+def test_row_major_ranges_hold_every_valid_scale_and_stay_inside_the_array(half):
+    """The same for row-major scales, whose rows may be further apart than their K/32 bytes (a column slice): the range
+    ends with the last valid row's bytes, whatever a 32-byte chunk asks for past them, on a whole dword."""
+    for stages in range(1, 10):
+        row = 8 * stages
+        for ld in (row, row + 4, row + 24, row + 32):
+            for rows in list(range(1, 40)) + [127, 128, 129, 255, 256, 257, 515]:
+                tile = 256 if half == 128 else half
+                size = (rows - 1) * ld + row  # the last row's padding need not exist
+                for base in range(0, -(-rows // tile) * tile, half):
+                    valid = min(max(rows - base, 0), half)
+                    end = (valid - 1) * ld + row if valid else 0
+                    assert end % 4 == 0 and (valid == 0 or base * ld + end <= size)
+                    assert valid == 0 or (valid - 1) * ld + row - 1 < end
