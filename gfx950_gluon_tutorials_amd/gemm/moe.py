@@ -14,8 +14,8 @@ layouts, with an expert dimension in front of B:
   [offsets[e], offsets[e + 1]) of A and C.
 
 C[t] = A[t] . B_e^T for every row t of expert e, computed by the same
-data-parallel tile as the dense kernels (one 256x256 tile per workgroup, 4
-waves), so each expert's rows are bit-identical to a dense ``matmul`` of that
+data-parallel tiles as the dense kernels (one tile per workgroup, 256x256 or, for
+few rows per expert, a small one), so each expert's rows are bit-identical to a dense ``matmul`` of that
 expert's slice.  Rows no expert owns are not written (with ``c=None`` they are
 left as ``torch.empty`` leaves them).  The launch is asynchronous on the
 current stream; the offsets are read on the device (no synchronisation).
@@ -28,7 +28,9 @@ import torch
 from .. import _lib
 from ._launch import _DTYPE_CODE, _OUT_CODE, _require_device, _stream
 
-KERNEL_NAME = "_moe_4w"
+# In the name of every grouped kernel (g9_*_moe_4w, and *_moe_t<rows>x<columns>
+# on small tiles) and of no other: the filter a profiler takes.
+KERNEL_NAME = "_moe_"
 
 
 def _offsets(expert_offsets: torch.Tensor, dev, E: int) -> torch.Tensor:

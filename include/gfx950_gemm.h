@@ -5,8 +5,8 @@
  * ("NT": A is M rows of K values, B is N rows of K values).  Three operand
  * types: FP16/BF16 (a16w16), BF8 = fp8 e5m2 with optional per-tensor fp32
  * scales (a8w8), and MXFP4 = e2m1 packed two per byte with one E8M0 scale per
- * 32 K-values (a4w4).  Three tile schedules: data-parallel (one 256x256 tile per
- * workgroup), stream-K (persistent workgroups over (tile, K-stage) work with
+ * 32 K-values (a4w4).  Three tile schedules: data-parallel (one tile per
+ * workgroup, 256x256 or, where that leaves the chip idle, smaller), stream-K (persistent workgroups over (tile, K-stage) work with
  * a K-ordered fp32 fixup; bit-identical to data-parallel) and split-K (for
  * grids of fewer tiles than half the CUs: each tile's K range is cut into
  * segments computed in parallel and their fp32 partials are summed in a fixed
@@ -248,12 +248,17 @@ int g9_moe_a4w4(const void* a, const void* b, void* c, const void* a_scales, con
                 int64_t stride_bn, int64_t stride_be, int64_t stride_asm, int64_t stride_bsn,
                 int64_t stride_bse, int64_t stride_cm, int out_dtype, void* stream);
 
-/* Name of the grouped kernel g9_moe_* launches for (dtype, out_dtype), or NULL. */
+/*
+ * Name of the grouped 256x256-tile kernel for (dtype, out_dtype), or NULL.
+ * Calls with few rows per expert launch a small-tile kernel instead,
+ * g9_<operands>_moe_t<rows>x<columns>: a profiler filter for both is "_moe_".
+ */
 const char* g9_moe_kernel_name(int dtype, int out_dtype);
 
 /*
  * Bytes of workspace a call with these arguments needs (0 for the
- * data-parallel schedule, and for split-K when it runs as data-parallel).
+ * data-parallel schedule, and for split-K when g9_splitk_factor is 1; a split-K
+ * call that takes small tiles asks for the split's).
  * `dtype` is the operand type.  Split-K's size depends on the current
  * device's CU count.  No counterpart in the reference (it has neither
  * stream-K nor split-K).
@@ -309,9 +314,12 @@ int g9_transpose_u8(const void* src, int64_t rows, int64_t cols, int64_t src_ld,
  * (16, `bf16` nonzero) or FP16 values.  MXFP4: `groups` groups of 32 values
  * to 16 bytes each of e2m1 codes (even value in the low nibble) and one E8M0
  * byte: E = floor(log2(largest magnitude)) - 2, codes rounded to nearest even
- * and saturated.  BF8: n values to e5m2 codes of x / scale with *scale =
- * largest magnitude / 57344 (1 for an all-zero tensor); `scratch` holds
- * G9_QUANT_SCRATCH_WORDS 4-byte words, written and read by the call.
+ * and saturated (where the device's pow(2, -E) falls below 2^-E, ties go to
+ * the smaller magnitude, as in x * pow(2, -E)).  BF8: n values to e5m2 codes of
+ * x / scale with *scale = largest magnitude * fp32(1 / 57344), which can differ
+ * in the last bit from the quotient, 1 for an all-zero or NaN tensor;
+ * `scratch` holds G9_QUANT_SCRATCH_WORDS 4-byte words, written and read by the
+ * call.
  */
 #define G9_QUANT_SCRATCH_WORDS 1024
 int g9_quantize_mxfp4(const void* x, int in_bits, int bf16, int64_t groups, void* packed, void* scales, void* stream);
@@ -319,11 +327,15 @@ int g9_quantize_e5m2(const void* x, int in_bits, int bf16, int64_t n, void* code
                      void* stream);
 
 /*
- * Name of the kernel a call with this (dtype, out_dtype, schedule, waves)
- * launches (for G9_SCHED_SPLITK: its segment kernel, followed by
- * g9_splitk_reduce_f16 or g9_splitk_reduce_bf16 by output type),
- * for profiler kernel filters (cf. KERNEL_NAME in
- * kernels/gemm/inter_wave/a8w8/matmul_kernel.py:52), or NULL.
+ * Name of the 256x256-tile kernel of this (dtype, out_dtype, schedule, waves)
+ * (for G9_SCHED_SPLITK: its segment kernel, followed by
+ * g9_splitk_reduce_f16 or g9_splitk_reduce_bf16 by output type), or NULL.
+ * Data-parallel calls whose 256x256 grid would leave the chip idle, and
+ * split-K calls that are faster so, launch a small-tile kernel instead,
+ * g9_<operands>_dp_t<rows>x<columns> for both output types.  A profiler filter
+ * for all of an operand type's kernels is its common prefix (g9_a16w16, g9_a8w8,
+ * g9_a4w4; cf. KERNEL_NAME in
+ * kernels/gemm/inter_wave/a8w8/matmul_kernel.py:52).
  */
 const char* g9_kernel_name(int dtype, int out_dtype, int schedule, int waves);
 
@@ -334,8 +346,9 @@ const char* g9_status_string(int status);
 int g9_streamk_workgroups(void);
 
 /*
- * K segments per tile the split-K schedule uses for `tiles` output tiles of
- * `stages` K stages on a device of `cus` CUs (1 = it runs as data-parallel).
+ * K segments per tile the split-K schedule uses, where it splits, for `tiles`
+ * output tiles of `stages` K stages on a device of `cus` CUs (1 = it runs as
+ * data-parallel; a call whose small tiles are faster does so at any factor).
  * Pure function of its arguments.  No counterpart in the reference.
  */
 int g9_splitk_factor(int64_t tiles, int stages, int cus);

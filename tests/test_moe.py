@@ -5,10 +5,13 @@ g9_capi.hip launch_moe) at every tile height, with up to and past one expert
 per lane, showing that any offset table keeps every access inside A, C and the
 experts' B, and that valid tables give each expert's rows to exactly one tile."""
 
+import re
+
 import numpy as np
 import pytest
 
 from gfx950_gluon_tutorials_amd import _lib
+from gfx950_gluon_tutorials_amd.gemm.moe import KERNEL_NAME
 
 FAKE = 0x10000
 
@@ -69,6 +72,14 @@ def test_moe_kernel_names():
              (_lib.G9_BF8, _lib.G9_F16), (_lib.G9_FP4, _lib.G9_BF16), (_lib.G9_FP4, _lib.G9_F16)]
     names = {_lib.moe_kernel_name(dt, out) for dt, out in pairs}
     assert len(names) == 6 and all(n and n.endswith("_moe_4w") for n in names)
+    # The profiler filter takes the grouped kernels of every tile, and only those.
+    with open(_lib.LIB_PATH, "rb") as fh:
+        built = {n.decode() for n in re.findall(rb"\bg9_[a-z0-9_]+(?:_[48]w|_t\d+x\d+)\b", fh.read())}
+    grouped = {n for n in built if KERNEL_NAME in n}
+    assert names | {f"g9_{op}_moe_t{tm}x{tn}" for op in ("a16w16_f16", "a16w16_bf16", "a8w8", "a4w4")
+                    for tm, tn in ((16, 16), (16, 32), (32, 32), (64, 32), (64, 64), (128, 64), (128, 128), (256, 128))} \
+        == grouped
+    assert not any("_dp_" in n or "_sk" in n or "_splitk_" in n for n in grouped)
     assert _lib.moe_kernel_name(_lib.G9_F16, _lib.G9_BF16) is None
 
 
