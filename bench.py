@@ -1011,7 +1011,9 @@ def main():
         codes = {"fp16": _lib.G9_F16, "bf8": _lib.G9_BF8, "mxfp4": _lib.G9_FP4}
         stage_k = {"fp16": 64, "bf8": 128, "mxfp4": 256}
         # Few-row GEMMs and one GPU's shard of a row-sharded 4096 x 4096 x 8192
-        # GEMM (512 rows = 1/8): 16-128 tiles, so data-parallel leaves CUs idle.
+        # GEMM (512 rows = 1/8): 16-128 256x256 tiles.  `split` is the factor of
+        # a call that splits; calls that are predicted faster on small tiles (then
+        # also what data-parallel runs, so the ratio is near 1) do not.
         for (dt, m, n, k) in [("fp16", 256, 4096, 8192), ("fp16", 512, 4096, 8192), ("fp16", 1024, 4096, 8192),
                               ("fp16", 2048, 4096, 8192), ("bf8", 512, 4096, 8192), ("mxfp4", 512, 4096, 8192)]:
             launch = make_case(dt, m, n, k, 5, dev, max(2, -(-args.rotate_mb * 2**20 // set_bytes(dt, m, n, k))))
@@ -1025,7 +1027,7 @@ def main():
                                            "splitk_tflops": round(flop / ms_sp / 1e9, 2), "dp_ms": round(ms_dp, 5),
                                            "splitk_ms": round(ms_sp, 5), "tiles": tiles, "split": S,
                                            "workspace_bytes": ws}
-            print(f"# split-K {dt} {m}x{n}x{k} ({tiles} tiles, {S} segments): dp {flop / ms_dp / 1e9:.1f}  "
+            print(f"# split-K {dt} {m}x{n}x{k} ({tiles} tiles, {S} segments or small tiles): dp {flop / ms_dp / 1e9:.1f}  "
                   f"splitk {flop / ms_sp / 1e9:.1f} TFLOPS ({ms_dp / ms_sp:.2f}x)", flush=True)
             del launch
             torch.cuda.empty_cache()
