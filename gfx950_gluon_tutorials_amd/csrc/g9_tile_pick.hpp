@@ -35,10 +35,10 @@ inline bool tile_addresses(int tm, long long lda, long long ldsa) {
 // 8192 x 512 and 5000 x 4096, K 512-14336, one MI355X (256 CUs), operands in
 // the 256 MB memory-side cache.  Over those shapes and the three types the tile
 // picked takes 0.2% longer than the fastest one on average, 10% at most; they
-// are the shapes of the fit.  Rows that are no whole number of 128-byte lines
-// apart take the small tiles up to twice as long as predicted, but of 240
-// drawn data-parallel calls with such rows (up to 600 256x256 tiles) none took
-// more than 3% longer than on 256x256 tiles.
+// are the shapes of the fit.  Stages that straddle two 128-byte lines (by the
+// rows' distance, their base or a K tail) take the small tiles up to twice as
+// long as predicted, but of 470 drawn data-parallel calls with such stages (up
+// to 600 256x256 tiles) none took more than 3% longer than on 256x256 tiles.
 struct TileCost {
   float fixed, stage;
 };
@@ -98,9 +98,9 @@ inline int pick_tile(const TileProblem& p) {
 }
 
 // Predicted time (us) of split-K with S segments for each of `tiles` 256x256
-// tiles: launches and a tile's fixed cost, a segment's stages (`ragged`: rows
-// that are no whole number of 128-byte lines apart), and a share per 256 KiB
-// partial of the reduction.  Least-squares fit to the split's times on 231
+// tiles: launches and a tile's fixed cost, a segment's stages (`ragged`: stages
+// of a row straddle two 128-byte lines), and a share per 256 KiB partial of the
+// reduction.  Least-squares fit to the split's times on 231
 // drawn shapes near the rule below (rms error 7%).
 constexpr float kSplitStage[3] = {1.16f, 1.12f, 1.35f};
 inline double splitk_time(int family, int ns, long long tiles, int S, bool ragged) {
@@ -114,7 +114,7 @@ inline double splitk_time(int family, int ns, long long tiles, int S, bool ragge
 // know, so the factors take the smallest geometric mean of both over the 231
 // shapes (0.3% above the better of the two on average): FP16/BF16 tiles, whose
 // predictions are up to 15% high, within 1.05 of the split, BF8 and MXFP4
-// below 0.88, and rows off 128-byte lines, which cost the tiles up to twice
+// below 0.88, and stages off 128-byte lines, which cost the tiles up to twice
 // their prediction, below 0.7.  Operands of more than 140 MB do not stay in
 // the cache from one call to the next.  None of the 231 then loses to the
 // split with its operands in the cache; with 1.0, 1.0 and 0.65 in their place

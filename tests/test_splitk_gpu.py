@@ -254,6 +254,40 @@ def test_splitk_random_shapes_match_dp(gpu, M, N, stages, waves, kind, splits):
         assert err <= 1e-3, f"relative Frobenius error {err:.3g} against data-parallel"
 
 
+@pytest.mark.parametrize("kind,M,N,K,tail,splits", [("fp16", 354, 4144, 9448, True, 7), ("bf16", 2071, 800, 10504, True, 7),
+                                                    ("fp16", 1731, 664, 6080, False, 12), ("bf8", 5169, 384, 19744, True, 6),
+                                                    ("bf8", 4174, 368, 14080, False, 7)])
+def test_stages_off_lines_stay_split(gpu, kind, M, N, K, tail, splits):
+    """Rows whole 128-byte lines apart whose stages still straddle two of them, by a K tail or by a base 16 bytes past a
+    line: the small tiles take up to 1.6 times the split's time there, so these split."""
+    _say(f"split-K {kind} {M}x{N}x{K} off lines by {'a K tail' if tail else 'the base'}")
+    es = 1 if kind == "bf8" else 2
+    line, off = 128 // es, 0 if tail else 16 // es
+    assert (K % line != 0) == tail
+    g = torch.Generator(device=gpu).manual_seed(M)
+
+    def operand(rows):
+        x = torch.randn(rows, K, generator=g, device=gpu) * 0.1
+        x = x.to(torch.float8_e5m2 if es == 1 else torch.float16 if kind == "fp16" else torch.bfloat16)
+        ld = -(-K // line) * line
+        v = torch.empty(rows * ld + off, dtype=x.dtype, device=gpu)[off:].as_strided((rows, K), (ld, 1))
+        return v.copy_(x)
+
+    a, b = operand(M), operand(N)
+    out = torch.bfloat16 if es == 1 else a.dtype
+    c, want = torch.empty(M, N, dtype=out, device=gpu), torch.empty(M, N, dtype=out, device=gpu)
+    (launched.a8w8 if es == 1 else launched.a16w16)(splits, a, b.T, c, schedule="splitk")
+    gemm = _launch.gemm_a8w8 if es == 1 else _launch.gemm_a16w16
+    gemm(a, b.T, c, schedule="splitk")
+    gemm(a, b.T, want)
+    torch.cuda.synchronize()
+    if es == 2:
+        _check_f16(c, want.float().cpu().numpy(), K, 0.01)
+    else:
+        err = R.rel_frobenius(c.float().cpu().numpy(), want.float().cpu().numpy())
+        assert err <= 1e-3, f"relative Frobenius error {err:.3g} against data-parallel"
+
+
 def test_splitk_through_the_drop_in_wrappers(gpu):
     """schedule="splitk" on the reference-shaped wrappers (4-wave a16w16 `matmul`,
     8-wave a4w4 `matmul_kernel_only`)."""

@@ -31,6 +31,21 @@ def test_splitk_calls_take_the_faster_side(problem, want):
     assert P.splitk(*problem) == want
 
 
+# Rows whole lines apart, but stages off them by the base (K whole lines) or by a K tail: us of the tile and of the split.
+OFF_LINES = [(("bf16", 1731, 664, 6080), 12),     # 47.2, 35.7
+             (("bf8", 4174, 368, 14080), 7),      # 57.1, 43.2
+             (("bf16", 354, 4144, 9448), 7),      # 69.6, 47.8
+             (("bf8", 5169, 384, 19744), 6)]      # 80.9, 56.6
+
+
+@pytest.mark.parametrize("problem,want", OFF_LINES)
+def test_stages_off_lines_stay_split(problem, want):
+    kind, K = problem[0], problem[3]
+    lda = -(-P._row(kind, K) // 128) * 128
+    assert P.splitk(*problem, lda=lda, off_line=True) == want
+    assert (P.splitk(*problem, lda=lda) == want) == (lda != P._row(kind, K))
+
+
 @pytest.mark.parametrize("kind", list(P.KINDS))
 def test_tiles_address_their_rows(kind):
     """From row strides of 2^23 bytes on the 256-row tile is no choice, and the next best one is

@@ -69,8 +69,9 @@ def factor(kind, M, N, K):
     return _lib.load().g9_splitk_factor(-(-M // 256) * -(-N // 256), -(-K // KINDS[kind][2]), CUS)
 
 
-def splitk(kind, M, N, K, lda=None):
-    """The segments per 256x256 tile of a split-K call, or the tile of the data-parallel launch it becomes."""
+def splitk(kind, M, N, K, lda=None, off_line=False):
+    """The segments per 256x256 tile of a split-K call, or the tile of the data-parallel launch it becomes; off_line:
+    the operands start off a 128-byte line."""
     family, value, stage = KINDS[kind]
     row = _row(kind, K)
     lda = row if lda is None else lda
@@ -78,7 +79,7 @@ def splitk(kind, M, N, K, lda=None):
     S = factor(kind, M, N, K)
     bytes_ = (M + N) * K * value + 2 * M * N
     shape = _pick().dense(family, M, N, ns, bytes_, lda, 0)
-    ragged = lda % 128 != 0 or row % 128 != 0
+    ragged = off_line or lda % 128 != 0 or row % 128 != 0  # (row: a K tail shifts every stage)
     if S <= 1 or _pick().beats(family, M, N, ns, bytes_, lda, shape, tiles, S, ragged):
         return _tile(shape)
     return S
